@@ -860,11 +860,6 @@ __device__ __forceinline__ u32x4_t asm_ldg128_nt(const uint8_t* base, uint32_t o
   asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(v) : "v"(off), "s"(base));
   return v;
 }
-__device__ __forceinline__ u32x4_t asm_ldg128(const uint8_t* base, uint32_t off) {
-  u32x4_t v;
-  asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(v) : "v"(off), "s"(base));
-  return v;
-}
 // Direct global -> LDS copy of 16 bytes per lane at base + off: lane l's bytes land at lds + 16 l.
 __device__ __forceinline__ void asm_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds) : "m0");
@@ -876,11 +871,13 @@ __device__ __align__(256) uint8_t exact_dummy_page[1024];
 
 // Exact-core LDS ring: kXStages stages of kStageChunks chunks each: the chunks' scale words (256 B each, 1 KB)
 // and, per token of the slot, the chunks' scaled activations (256 B each, 1 KB per token); xstage_bytes(T)
-// with the call's token count T bounding every slot's. The ring lives in the launch's dynamic LDS.
+// with the call's token count T bounding every slot's. The ring lives in the launch's dynamic LDS. Token rows
+// are kXStageTok bytes apart, 16 more than a power of two, so that the 16-byte reads of several tokens' same
+// K block fall into different banks.
 constexpr int kStageChunks = 4;
 constexpr int kXStages = 2;
-constexpr int kXStageScale = 0, kXStageAct = 1024;
-__host__ __device__ constexpr int xstage_bytes(int T) { return 1024 + 1024 * T; }
+constexpr int kXStageScale = 0, kXStageAct = 1024, kXStageTok = 1024 + 16;
+__host__ __device__ constexpr int xstage_bytes(int T) { return kXStageAct + kXStageTok * T; }
 
 // Stage g's shared operands (chunks 4g .. 4g + 3) into ring slot st, one 1 KB copy instruction each: the scale
 // words, and one per token (token j by wave j % 4, the scale words by wave ntok % 4). In a last stage holding
@@ -902,18 +899,14 @@ struct SharedCopies {
   __device__ __forceinline__ int copies() const { return n_act + (copies_scale ? 1 : 0); }
   __device__ __forceinline__ void issue(int g, int st) const {
     const uint32_t base = lds + st * stage_bytes;
-    if (kStageChunks * g < n) {
-      const uint32_t k = (int)lane < 16 * (n - kStageChunks * g) ? (uint32_t)g * 1024 + 16 * lane : 0;
-      if (copies_scale) asm_copy16(scale, k, base + kXStageScale);
+    const int left = n - kStageChunks * g;   // the row's chunks from this stage on
+    const uint8_t* sbase = left > 0 ? scale : dummy;
+    const uint8_t* abase = left > 0 ? act : dummy;
+    const uint32_t k = left <= 0 ? 16 * lane : (int)lane < 16 * left ? (uint32_t)g * 1024 + 16 * lane : 0;
+    if (copies_scale) asm_copy16(sbase, k, base + kXStageScale);
 #pragma unroll
-      for (int i = 0; i < kMaxTokens / 4; ++i)
-        if (i < n_act) asm_copy16(act, act_row[i] + k, base + kXStageAct + 1024 * act_tok[i]);
-    } else {
-      if (copies_scale) asm_copy16(dummy, 16 * lane, base + kXStageScale);
-#pragma unroll
-      for (int i = 0; i < kMaxTokens / 4; ++i)
-        if (i < n_act) asm_copy16(dummy, 16 * lane, base + kXStageAct + 1024 * act_tok[i]);
-    }
+    for (int i = 0; i < kMaxTokens / 4; ++i)
+      if (i < n_act) asm_copy16(abase, (left > 0 ? act_row[i] : 0) + k, base + kXStageAct + kXStageTok * act_tok[i]);
   }
 };
 
@@ -944,50 +937,64 @@ __device__ __forceinline__ void transpose_groups(uint32_t (&v)[4]) {
   v[3] = d[1];
 }
 
-// Stage st's operands of this lane, read and waited for: the activations of blocks 0..3 at K 8 g (token column
-// n, or the slot's first token for idle columns) and the E8M0 codes of row m, blocks 0..3 (byte t of scale
-// word m + 16 b).
-__device__ __forceinline__ void lds_read_stage(uint32_t xaddr, uint32_t caddr, u32x4_t (&xb)[4], uint32_t (&code)[4]) {
-  asm volatile(
-      "ds_read_b128 %0, %8\n\t"
-      "ds_read_b128 %1, %8 offset:64\n\t"
-      "ds_read_b128 %2, %8 offset:128\n\t"
-      "ds_read_b128 %3, %8 offset:192\n\t"
-      "ds_read_u8 %4, %9\n\t"
-      "ds_read_u8 %5, %9 offset:64\n\t"
-      "ds_read_u8 %6, %9 offset:128\n\t"
-      "ds_read_u8 %7, %9 offset:192\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(xb[0]), "=&v"(xb[1]), "=&v"(xb[2]), "=&v"(xb[3]), "=&v"(code[0]), "=&v"(code[1]), "=&v"(code[2]),
-        "=&v"(code[3])
-      : "v"(xaddr), "v"(caddr));
-}
+typedef __attribute__((address_space(3))) const uint8_t* lds_u8_ptr;
+typedef __attribute__((address_space(3))) const u32x4_t* lds_u32x4_ptr;
 
-// Multiply chunk c (this lane's 16 weight bytes wa, LDS stage operands) into the chains.
-__device__ __forceinline__ void exact_chunk(const u32x4_t& wa, const u32x4_t (&xb)[4], const uint32_t (&code)[4],
-                                            v4f& acc) {
-  uint32_t wv[4] = {wa.x, wa.y, wa.z, wa.w};
-  transpose_groups(wv);   // lane group g now holds word g of every block: K 32 (4c + b) + 8 g + 0..7 in wv[b]
+// Tokens of a slot up to which the chunk's four blocks share the MFMA's token columns (exact_chunk_few).
+constexpr int kFewTokens = 4;
+
+// Multiply one chunk (transposed weights wv: lane group g holds word g of block b, K 32 (4c + b) + 8 g + 0..7, in
+// wv[b]) into the chains. xaddr / caddr: this lane's LDS addresses of
+// the chunk's activations and of its row's scale byte of block 0 (block b's is 64 b further). The reads are plain
+// LDS loads (the copies that filled the stage are inline assembly the compiler does not wait for; the stage's own
+// wait and barrier order them), so the compiler starts a chunk's reads under the previous chunk's work.
+//
+// Many tokens: column n is token n, MFMA b multiplies block b of all 16 tokens (four 16-byte reads), and
+// acc = acc + d runs in place.
+__device__ __forceinline__ void exact_chunk_many(const uint32_t (&wv)[4], uint32_t xaddr, uint32_t caddr, v4f& acc) {
+  const lds_u32x4_ptr px = (lds_u32x4_ptr)(size_t)xaddr;
+  const lds_u8_ptr pc = (lds_u8_ptr)(size_t)caddr;
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
-    const v8bf av = fp4_word_bits(wv[b], fp4_scale_float_bits(code[b]));
-    const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(v8bf, xb[b]),
+    const v8bf av = fp4_word_bits(wv[b], fp4_scale_float_bits(pc[64 * b]));
+    const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(v8bf, px[4 * b]),
                                                           v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = acc[i] + d[i];
   }
 }
 
-// The whole K range (n chunks) of tile `wave` of a row group, stage by stage. At the
-// start of stage g a wave waits until its own copies of stage g have landed, a barrier makes every wave's copies
-// visible, and the wave issues its copies of stage g + kXStages - 1 (into the ring slot of stage g - 1, which
-// every wave finished reading before this barrier); then for each chunk c of the stage it reads the chunk's
-// operands from LDS, multiplies chunk c and issues its weights for chunk c + kW. kW = kXStages x kStageChunks,
-// so the weights of a stage's chunks are issued before that stage's copies, and past the end weights load from
-// the dummy page and copies read it: every stage issues the same loads per wave, and when a wave waits for its
-// copies of stage g, the loads issued after them -- the weights of stage g - kXStages + 1's chunks and, per
-// later stage, copies + kStageChunks weights -- may still be in flight.
-constexpr int kWRing = kXStages * kStageChunks;
+// Up to kFewTokens tokens, operands exchanged: A is the activations, its row 4 t + b block b of token t, so ONE
+// 16-byte read per chunk is the operand of all four MFMAs, and B is the weights (column n = weight row n). MFMA b
+// multiplies block b's weights; of its D (lane (n, g) register i = activation row 4 g + i = token g, block i)
+// register b holds that block's dots, the other three multiply unrelated blocks and are dropped. So lane (n, g)
+// keeps the one chain of weight row n and token g, and a chunk takes four additions instead of sixteen. Nearly all
+// slots of a decode call hold this few tokens. What bounds the kernel is the weight stream once its waves' own work
+// (conversions, additions, LDS reads) stays below it: with one form for all token counts (a column per token, four
+// LDS reads and sixteen additions a chunk) gate/up of the 7168 x 2048 layer took 84 us at 4 tokens and 255 us at 16
+// (5.6 and 6.5 TB/s, re-launched on one layer), now 78 and 239 us (6.0 and 6.9 TB/s; the plain read kernel 7.0);
+// one token 31.1 -> 29.5 us.
+__device__ __forceinline__ float exact_chunk_few(const uint32_t (&wv)[4], uint32_t xaddr, uint32_t caddr, float acc) {
+  const v8bf xa = __builtin_bit_cast(v8bf, *(lds_u32x4_ptr)(size_t)xaddr);
+  const lds_u8_ptr pc = (lds_u8_ptr)(size_t)caddr;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, fp4_word_bits(wv[b], fp4_scale_float_bits(pc[64 * b])),
+                                                          v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    acc = acc + d[b];
+  }
+  return acc;
+}
+
+// The whole K range (n chunks) of tile `wave` of a row group, stage by stage. At the start of stage g a wave waits
+// until its weights and its own copies of stage g have landed, a barrier makes every wave's copies visible, and the
+// wave issues its copies of stage g + kX - 1 (into the ring slot of stage g - 1, which every wave finished reading
+// before this barrier) and, once the stage's weights have left their ring slots, its weights of stage g + kWS; then
+// it multiplies the stage's chunks. Past the end weights load from the dummy page and copies read it, so every stage
+// issues the same loads per wave. When a wave waits at stage g, what it issued after the weights of stage g (stages
+// g - kWS + 1 .. g - 1: copies + kStageChunks loads each) and after its copies of stage g (the weights of stage
+// g - kX + 1 and all of the later stages) may still be in flight.
+constexpr int kWStages = 2;   // stages of weights in the register ring
 
 template <int kAfter>
 __device__ __forceinline__ void vm_wait() {
@@ -995,60 +1002,81 @@ __device__ __forceinline__ void vm_wait() {
   __builtin_amdgcn_s_waitcnt(mxd::vm_wait_imm(kAfter));
 }
 
-// wait for this wave's copies of a stage, with `copies` copy instructions per stage (0 .. 5)
-template <int kCopies>
+// wait for this wave's weights and copies of a stage, with `copies` copy instructions per stage (0 .. 5)
+template <int kX, int kCopies>
 __device__ __forceinline__ void wait_stage() {
-  vm_wait<kStageChunks + (kXStages - 2) * (kCopies + kStageChunks)>();
+  constexpr int kPer = kCopies + kStageChunks;
+  constexpr int kAfterW = (kWStages - 1) * kPer, kAfterC = kStageChunks + (kX - 2) * kPer;
+  vm_wait<(kAfterW < kAfterC ? kAfterW : kAfterC)>();
 }
 
+template <bool kFew, int kX>
 __device__ __forceinline__ void stream_exact(const uint8_t* wbase, uint32_t woff, const SharedCopies& sc,
                                              uint32_t xaddr, uint32_t caddr, int n, v4f& acc) {
-  constexpr int kW = kWRing, kX = kXStages, kC = kStageChunks;
+  constexpr int kC = kStageChunks, kWS = kWStages, kW = kWS * kC;
   const int sb = sc.stage_bytes, n_stages = (n + kC - 1) / kC, copies = sc.copies();
   acc = v4f{0.f, 0.f, 0.f, 0.f};
   u32x4_t wr[kW];
-  auto load_w = [&](u32x4_t& r, int c) {
-    if (c < n) r = asm_ldg128_nt(wbase + (size_t)c * 4096, woff);
-    else r = asm_ldg128(sc.dummy, 16 * sc.lane);
-  };
-  // the loads of stages -kX .. -1 in the steady state's order: stage g issues C(g + kX - 1) (when that stage
-  // index is not negative), then the weights of chunks kC g + kW .. kC g + kW + kC - 1
+  // past the last chunk the base is the dummy page (woff is 16 x lane), selected without a branch
+  auto load_w = [&](u32x4_t& r, int c) { r = asm_ldg128_nt(c < n ? wbase + (size_t)c * 4096 : sc.dummy, woff); };
+  // the loads of the stages before 0 in the steady state's order: stage g issues C(g + kX - 1), then W(g + kWS)
+  // (those whose stage index is negative do not exist)
+  constexpr int kPro = kWS > kX - 1 ? kWS : kX - 1;
 #pragma unroll
-  for (int vg = -kX; vg < 0; ++vg) {
-    if (vg + kX - 1 >= 0) sc.issue(vg + kX - 1, (vg + kX - 1) % kX);
+  for (int vg = -kPro; vg < 0; ++vg) {
+    if (vg + kX - 1 >= 0) sc.issue(vg + kX - 1, vg + kX - 1);
+    if (vg + kWS >= 0) {
 #pragma unroll
-    for (int u = 0; u < kC; ++u) load_w(wr[kC * (vg + kX) + u], kC * vg + kW + u);
+      for (int u = 0; u < kC; ++u) load_w(wr[kC * (vg + kWS) + u], kC * (vg + kWS) + u);
+    }
   }
-  for (int g0 = 0; g0 < n_stages; g0 += kX) {
+  int slot = 0;   // g % kX
+  for (int g0 = 0; g0 < n_stages; g0 += kWS) {
 #pragma unroll
-    for (int gs = 0; gs < kX; ++gs) {
+    for (int gs = 0; gs < kWS; ++gs) {
       const int g = g0 + gs;
       // the waits and ties run for every slot, past the end too: a slot's registers are only released (and
       // reusable by the compiler) once the load that writes them has landed
       switch (copies) {
-        case 0: wait_stage<0>(); break;
-        case 1: wait_stage<1>(); break;
-        case 2: wait_stage<2>(); break;
-        case 3: wait_stage<3>(); break;
-        case 4: wait_stage<4>(); break;
-        default: wait_stage<5>(); break;
+        case 0: wait_stage<kX, 0>(); break;
+        case 1: wait_stage<kX, 1>(); break;
+        case 2: wait_stage<kX, 2>(); break;
+        case 3: wait_stage<kX, 3>(); break;
+        case 4: wait_stage<kX, 4>(); break;
+        default: wait_stage<kX, 5>(); break;
       }
 #pragma unroll
       for (int u = 0; u < kC; ++u) asm volatile("" : "+v"(wr[kC * gs + u]));   // landed with the wait above
       // every wave's copies of stage g have landed, and every wave has finished reading stage g - 1, whose slot
       // this stage's copies overwrite (past the last stage only that one is still read)
       if (g <= n_stages) mxd::copy_barrier();
-      sc.issue(g + kX - 1, (gs + kX - 1) % kX);
+      sc.issue(g + kX - 1, slot == 0 ? kX - 1 : slot - 1);
+      // the stage's weights leave the ring transposed, and its slots take their next loads at once: no register
+      // with a load in flight is touched again, nor merged from two paths, before the wait that ties it
+      uint32_t wv[kC][4];
 #pragma unroll
       for (int u = 0; u < kC; ++u) {
-        const int c = kC * g + u;
-        if (c < n) {
-          u32x4_t xb[4];
-          uint32_t code[4];
-          lds_read_stage(xaddr + gs * sb + 256 * u, caddr + gs * sb + 256 * u, xb, code);
-          exact_chunk(wr[kC * gs + u], xb, code, acc);
+        const u32x4_t& r = wr[kC * gs + u];
+        wv[u][0] = r.x, wv[u][1] = r.y, wv[u][2] = r.z, wv[u][3] = r.w;
+        transpose_groups(wv[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kC; ++u) load_w(wr[kC * gs + u], kC * g + u + kW);
+      const uint32_t xs = xaddr + slot * sb, cs = caddr + slot * sb;
+      slot = slot == kX - 1 ? 0 : slot + 1;
+      if (kC * g + kC <= n) {   // a whole stage: no branches between its chunks
+#pragma unroll
+        for (int u = 0; u < kC; ++u) {
+          if constexpr (kFew) acc[0] = exact_chunk_few(wv[u], xs + 256 * u, cs + 256 * u, acc[0]);
+          else exact_chunk_many(wv[u], xs + 256 * u, cs + 256 * u, acc);
         }
-        load_w(wr[kC * gs + u], c + kW);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kC; ++u)
+          if (kC * g + u < n) {
+            if constexpr (kFew) acc[0] = exact_chunk_few(wv[u], xs + 256 * u, cs + 256 * u, acc[0]);
+            else exact_chunk_many(wv[u], xs + 256 * u, cs + 256 * u, acc);
+          }
       }
     }
   }
@@ -1169,59 +1197,36 @@ __device__ __forceinline__ v4f reduce_tiles(const v4f (&acc)[kTiles], int wave, 
   return out;
 }
 
-// SwiGLU epilogue of gate/up tile t of row group g: in `mine` (the in-order chains), lane (n, q) holds token
-// column n; lanes with q < 2 hold W1 rows 4q + i of the tile (D[4q + i][n]) and lane + 32 the matching W3
-// rows. Writes the down input of token n to s_din[n][8t + 4q + i] (and the diagnostic copies when requested).
-__device__ __forceinline__ void gateup_tile_epilogue(const ExpertArgs& a, const SlotView& sv, int g, int t,
-                                                     const v4f& mine, int lane, int ntok, float (*s_din)[32]) {
-  float upv[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) upv[i] = __shfl_xor(mine[i], 32, 64);
-  const int q = lane >> 4, n = lane & 15;
-  if (q < 2 && n < ntok) {
-    const int row0 = sv.row0;
-    const bool weighted = sv.weighted != 0;
-    const float rw = sv.w[n];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int li = t * 8 + 4 * q + i;           // row within the 32-row block
-      const int gi = g * 32 + li;                 // intermediate index
-      const uint32_t b1 = mx::bf16_bits(mine[i]);
-      const uint32_t b3 = mx::bf16_bits(upv[i]);
-      const size_t o2 = (size_t)(row0 + n) * a.I + gi;
-      const float din = mxd::swiglu_element(b1, b3, a.limit, weighted, rw, a.trace ? a.trace + o2 * 5 : nullptr);
-      s_din[n][li] = din;
-      if (a.w1) a.w1[o2] = (uint16_t)b1;
-      if (a.w3) a.w3[o2] = (uint16_t)b3;
-      if (a.din) a.din[o2] = (uint16_t)mx::bf16_bits(din);
-    }
+// Epilogue of a gate/up workgroup, on row group g's 32 W1 and 32 W3 sums of every token (FP32, in s_gu): thread
+// (token, row) applies SwiGLU to its element, and the token's 32 threads quantize its block of the down input (one
+// E8M0 block). One element per thread: the float64 exp of silu_f32 is a chain of dependent instructions, which
+// four elements per lane of one wave paid four times over.
+__device__ __forceinline__ void gateup_epilogue(const ExpertArgs& a, const SlotView& sv, int g, int ntok,
+                                                const float (*s_gu)[kMaxTokens][36]) {
+  for (int p = threadIdx.x; p < 32 * ntok; p += 256) {
+    const int tok = p >> 5, li = p & 31, gi = g * 32 + li;
+    const size_t row = (size_t)(sv.row0 + tok), o = row * a.I + gi;
+    const uint32_t b1 = mx::bf16_bits(s_gu[0][tok][li]), b3 = mx::bf16_bits(s_gu[1][tok][li]);
+    const float din = mxd::swiglu_element(b1, b3, a.limit, sv.weighted != 0, sv.w[tok], a.trace ? a.trace + o * 5 : nullptr);
+    if (a.w1) a.w1[o] = (uint16_t)b1;
+    if (a.w3) a.w3[o] = (uint16_t)b3;
+    if (a.din) a.din[o] = (uint16_t)mx::bf16_bits(din);
+    float amax = mxd::row16_max(fabsf(din));
+    amax = fmaxf(fmaxf(amax, __shfl_xor(amax, 16, 32)), mx::u2f(mx::kAmaxFloorBits));
+    const uint32_t code = mx::act_scale_code(amax);
+    a.dq[o] = (uint8_t)mx::act_quant_pow2(din, 1.0f / mx::e8m0_value(code));   // exact: a power of two
+    if (li == 0) a.ds[row * (a.I / 32) + g] = (uint8_t)code;
   }
-}
-
-// Per-token quantization of row group g's 32-row block of the down input (one E8M0 block per token):
-// 16 consecutive threads j2 = 0..15 take token tn, 2 values each.
-__device__ __forceinline__ void gateup_quantize_block(const ExpertArgs& a, const SlotView& sv, int g, int tn, int j2,
-                                                      int ntok, const float (*s_din)[32]) {
-  if (tn >= ntok) return;
-  const int I = a.I;
-  const float v0 = s_din[tn][2 * j2], v1 = s_din[tn][2 * j2 + 1];
-  float amax = mxd::row16_max(fmaxf(fabsf(v0), fabsf(v1)));   // the token's 16 lanes are one row
-  amax = fmaxf(amax, mx::u2f(mx::kAmaxFloorBits));
-  const uint32_t code = mx::act_scale_code(amax);
-  const float sc = mx::e8m0_value(code);
-  const float inv = 1.0f / sc;   // exact: sc is a power of two
-  const uint32_t q0 = mx::act_quant_pow2(v0, inv), q1 = mx::act_quant_pow2(v1, inv);
-  const size_t r = (size_t)(sv.row0 + tn);
-  *reinterpret_cast<uint16_t*>(a.dq + r * I + g * 32 + 2 * j2) = (uint16_t)(q0 | (q1 << 8));
-  if (j2 == 0) a.ds[r * (I / 32) + g] = (uint8_t)code;
 }
 
 // One-token decode, routing folded into gate/up: wave 0 selects the token's k experts from the router's
 // selection values and scores (topk_token_wave, the same selection and weights as route_plan_kernel), and
 // slot s is the selected expert with s smaller selected IDs (row s, the token's route weight), or the shared
 // expert for s = k (row k) -- route_plan_kernel's plan for one token, where pairs run expert-major. Workgroup
-// (0, 0) also writes the routing outputs and the plan itself (build_plan) for the down and combine launches
-// that follow on the stream; every workgroup computes the same selection from the same inputs.
+// (0, 0) also writes the routing outputs and the plan itself (build_plan) for the launches that follow on the
+// stream; every workgroup computes the same selection from the same inputs. (A workgroup of its own for the
+// outputs and the plan measured the same, and one more column of workgroups 2 us slower: the rows of the grid
+// then no longer fall evenly on the 8 XCDs.)
 __device__ void select_slot_one_token(const ExpertArgs& a, int s, SlotView& sv) {
   __shared__ int32_t s_idx[kMaxTopK];
   __shared__ float s_w[kMaxTopK];
@@ -1245,26 +1250,22 @@ __device__ void select_slot_one_token(const ExpertArgs& a, int s, SlotView& sv) 
     sv.n_slots = a.k + a.has_shared;
     sv.ntok = 1;
     sv.tok[0] = 0;
-    if (s < a.k) {
-      int e = 0;
-      float w = 0.f;
-      for (int j = 0; j < a.k; ++j) {
-        int below = 0;
-        for (int i = 0; i < a.k; ++i) below += s_idx[i] < s_idx[j];
-        if (below == s) {
-          e = s_idx[j];
-          w = s_w[j];
-        }
-      }
-      sv.expert = e;
-      sv.row0 = s;
-      sv.weighted = 1;
-      sv.w[0] = w;
-    } else {
+    if (s == a.k) {
       sv.expert = a.E;
       sv.row0 = a.k;
       sv.weighted = 0;
       sv.w[0] = 1.0f;
+    }
+  }
+  if (s < a.k && threadIdx.x < a.k) {   // thread j holds the token's j-th expert: it is slot s's if s are smaller
+    const int e = s_idx[threadIdx.x];
+    int below = 0;
+    for (int i = 0; i < a.k; ++i) below += s_idx[i] < e;
+    if (below == s) {
+      sv.expert = e;
+      sv.row0 = s;
+      sv.weighted = 1;
+      sv.w[0] = s_w[threadIdx.x];
     }
   }
   __syncthreads();
@@ -1303,10 +1304,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
   if (s >= sv.n_slots) return;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane >> 4, m = lane & 15, n = lane & 15;
-  const int ntok = sv.ntok;
+  // the slot's values come from LDS: made scalar, so that the core's bases and conditions are
+  const int ntok = __builtin_amdgcn_readfirstlane(sv.ntok);
   const int H = a.H, I = a.I;
   const size_t chunks = H / 128;
-  const uint8_t* blob = a.tiles[sv.expert];
+  const uint8_t* blob = a.tiles[__builtin_amdgcn_readfirstlane(sv.expert)];
   extern __shared__ __attribute__((aligned(16))) uint8_t ring[];   // kXStages x xstage_bytes(a.tokens)
   const uint32_t ring0 = mxd::lds_addr(ring);
   SharedCopies sc;
@@ -1317,7 +1319,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
   for (int i = 0; i < kMaxTokens / 4; ++i) {   // tokens wave, wave + 4, ... of the slot
     const int j = wave + 4 * i;
     sc.act_tok[i] = j;
-    sc.act_row[i] = (uint32_t)sv.tok[j < ntok ? j : 0] * (uint32_t)(2 * H);
+    sc.act_row[i] = (uint32_t)__builtin_amdgcn_readfirstlane(sv.tok[j < ntok ? j : 0]) * (uint32_t)(2 * H);
     if (j < ntok) sc.n_act = i + 1;
   }
   sc.dummy = exact_dummy_page;
@@ -1326,17 +1328,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
   sc.lds = ring0;
   sc.stage_bytes = xstage_bytes(a.tokens);
   sc.copies_scale = wave == (ntok & 3);
-  // this lane's LDS operands: token column n's row (the slot's first token for idle columns) at K 8 q, and the
+  // this lane's LDS operands: its column's token row (the slot's first token for idle columns) at K 8 q, and the
   // scale byte of tile `wave` for row m (word m + 16 b holds block b)
-  const uint32_t xaddr = ring0 + kXStageAct + 1024 * (n < ntok ? n : 0) + 16 * q;
+  // (few tokens: block n % 4 of token n / 4)
+  const bool few = kPlanInGateup || ntok <= kFewTokens;
+  const int tok = few ? n >> 2 : n;   // the token of this lane's activations
+  const uint32_t xaddr = ring0 + kXStageAct + kXStageTok * (tok < ntok ? tok : 0) + 16 * q + (few ? 64 * (n & 3) : 0);
   const uint32_t caddr = ring0 + kXStageScale + 4 * m + wave;
   const uint8_t* wbase = blob + (size_t)g * chunks * 4096 + (size_t)wave * 1024;
   v4f acc;
-  stream_exact(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
-  __shared__ float s_din[kMaxTokens][32];
-  gateup_tile_epilogue(a, sv, g, wave, acc, lane, ntok, s_din);
+  if (few) stream_exact<true, kXStages>(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
+  else stream_exact<false, kXStages>(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
+  // tile `wave` holds the group's W1 rows 8 wave + 0..7 as rows 0-7 and the same W3 rows as rows 8-15: lane (n, q)
+  // has token n's sums of tile rows 4q + i, or with few tokens token q's sum of tile row n
+  __shared__ __attribute__((aligned(16))) float s_gu[2][kMaxTokens][36];
+  if (few) {
+    if (q < ntok) s_gu[n >> 3][q][8 * wave + (n & 7)] = acc[0];
+  } else if (n < ntok) {
+    *reinterpret_cast<v4f*>(&s_gu[q >> 1][n][8 * wave + 4 * (q & 1)]) = acc;
+  }
   __syncthreads();
-  gateup_quantize_block(a, sv, g, tid >> 4, tid & 15, ntok, s_din);
+  gateup_epilogue(a, sv, g, ntok, s_gu);
 }
 
 // Output rows [64b, 64b + 64) of slot s's W2 as 4 tiles of 16 rows; after the cross-wave sum wave t writes
