@@ -80,38 +80,6 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
-// Device-coherent 8-byte store and load: agent-scope relaxed atomics, which gfx950 issues with the sc1
-// scope bit, so the store is written through to the device's coherence point and the load does not hit a
-// stale line of this XCD's L2. Workgroups on different XCDs exchange data this way without the whole-L2
-// write-back and invalidate that an agent-scope fence costs.
-__device__ __forceinline__ void store_device(float* p, float a, float b) {
-  const uint64_t v = (uint64_t)__float_as_uint(a) | ((uint64_t)__float_as_uint(b) << 32);
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ float2 load_device(const float* p) {
-  const uint64_t v =
-      __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
-}
-
-// Handoff buffers between workgroups (the split-K GEMV's partial sums) hold this FP32 pattern wherever no
-// value is published: a signalling NaN, which FP32 arithmetic never produces (its NaN results are quiet).
-constexpr uint32_t kHandoffEmpty = 0x7FA0DEADu;
-constexpr int kHandoffPolls = 1 << 16;
-
-// The pair `first` read from p, re-read until it is no longer the empty pattern (a pair is published by one
-// 64-bit atomic, so its halves arrive together); at most kHandoffPolls reads, then NaN instead of a hang.
-__device__ __forceinline__ float2 await_pair(float2 first, const float* p) {
-  float2 v = first;
-  for (int i = 0; __float_as_uint(v.x) == kHandoffEmpty; ++i) {
-    if (i == kHandoffPolls) return make_float2(__builtin_nanf(""), __builtin_nanf(""));
-    __builtin_amdgcn_s_sleep(1);
-    v = load_device(p);
-  }
-  return v;
-}
-
 // V_MFMA_SCALE_F32_16X16X128_F8F6F4 operand layouts (measured on gfx950 with one-hot probes):
 //   FP4 A (cbsz 4, 4 VGPRs): lane l = row l % 16, K = 32 (l / 16) + nibble j, low nibble first.
 //   FP8 A (cbsz 0) and FP8 B (blgp 0), 8 VGPRs: lane l = row / column l % 16; bytes 0-15 hold

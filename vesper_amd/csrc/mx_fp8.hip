@@ -34,11 +34,6 @@ using mxd::v4f;
 constexpr int kTiles = 4;   // 16-row MFMA tiles per workgroup: 64 weight rows
 constexpr int kTok = 16;    // token columns per MFMA
 constexpr int kGemvMaxTokens = 32;   // above this the tiled GEMM reuses each weight tile for 128 tokens
-// The GEMV's last workgroup per tile adds the split-K partial sums when they total at most this many
-// bytes. Above it (the 7168- and 24576-row projections at 16 tokens, measured on MI355X) the
-// device-coherent round trip through one workgroup per tile costs more than fp8_splitk_reduce_kernel.
-constexpr uint64_t kTicketPartialBytes = MX_HANDOFF_BYTES;   // the context's handoff buffer
-
 struct Fp8Blob {
   size_t scales;   // byte offset of the scale section
   size_t total;    // blob bytes (256-byte multiple)
@@ -142,6 +137,57 @@ __global__ __launch_bounds__(256) void act_quant128_v8_kernel(const uint16_t* __
   }
 }
 
+// The 8 codes of this lane's values `raw` (one 128-value block per 16 lanes, sub = lane % 16) with the quantizer
+// launches' arithmetic, and their scale: block 32 the E8M0 code (the four lanes of a quad hold one), block 128 the
+// FP32 bits.
+template <int kBlock>
+__device__ __forceinline__ uint2 quantize8(const uint4& raw, uint32_t& scale) {
+  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+  float v[8];
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = mx::bf16_value(w[i] & 0xFFFFu);
+    v[2 * i + 1] = mx::bf16_value(w[i] >> 16);
+    amax = fmaxf(amax, fmaxf(fabsf(v[2 * i]), fabsf(v[2 * i + 1])));
+  }
+  if constexpr (kBlock == 32) {
+    amax = fmaxf(mxd::quad_max(amax), mx::u2f(mx::kAmaxFloorBits));
+    scale = mx::act_scale_code(amax);
+    const float r = 1.0f / mx::e8m0_value(scale);   // exact: a power of two
+    return make_uint2(mxd::e4m3x4(v[0] * r, v[1] * r, v[2] * r, v[3] * r),
+                      mxd::e4m3x4(v[4] * r, v[5] * r, v[6] * r, v[7] * r));
+  } else {
+    const float sc = mx::act128_scale(mxd::row16_max(amax));
+    scale = __float_as_uint(sc);
+    return act128_codes8(v, sc);
+  }
+}
+
+// Quantizer of the decode GEMV's own input: codes in the order in which its waves load them, so that a chunk's
+// operand of 16 tokens is two linear 1 KB loads instead of 32 row pieces of 64 bytes, and its scales 64 contiguous
+// bytes instead of 16 rows. Token tile tt (16 tokens), chunk c: half h of lane (q, n) -- token 16 tt + n, K 64 h + 16 q
+// + 0..15 of the chunk -- at (tt C + c) 2048 + 1024 h + 16 (16 q + n); the scales (block 32: four E8M0 codes, block 128:
+// FP32) at (tt C + c) 64 + 4 n. 16 lanes per (token, chunk).
+template <int kBlock>
+__global__ __launch_bounds__(256) void fp8_quant_ordered_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ q,
+                                                                uint8_t* __restrict__ s, int T, int C) {
+  const int b = (blockIdx.x * 256 + threadIdx.x) >> 4, sub = threadIdx.x & 15;
+  if (b >= T * C) return;   // whole groups of 16 lanes
+  const int t = b / C, c = b - t * C, n = t & 15;
+  uint32_t scale;
+  const uint2 codes =
+      quantize8<kBlock>(ldg128(reinterpret_cast<const uint8_t*>(x + ((size_t)t * C + c) * 128 + 8 * sub)), scale);
+  const size_t at = (size_t)(t >> 4) * C + c;
+  // values 8 sub .. 8 sub + 7: half sub / 8, lane group (sub / 2) % 4, upper or lower 8 bytes by sub % 2
+  *reinterpret_cast<uint2*>(q + at * 2048 + 1024 * (sub >> 3) + 16 * (16 * ((sub >> 1) & 3) + n) + 8 * (sub & 1)) = codes;
+  if constexpr (kBlock == 32) {
+    if ((sub & 3) == 0) s[at * 64 + 4 * n + (sub >> 2)] = (uint8_t)scale;
+  } else {
+    if (sub == 0) *reinterpret_cast<uint32_t*>(s + at * 64 + 4 * n) = scale;
+  }
+}
+
 struct Fp8Args {
   const uint8_t* blob;
   int N, K, T;
@@ -149,307 +195,178 @@ struct Fp8Args {
   const void* xs;      // block 32: uint8 [T][K/32]; block 128: float [T][K/128]
   uint16_t* y;         // [T][N] BF16
   float* trace;        // [T][N] FP32 sums, nullable
-  float* partial;      // split K: [splits][T][N] FP32 partial sums (the GEMV writes these instead of y)
-  uint32_t* tickets;   // split-K GEMV: arrival counter per (row group, token tile), zero between launches;
-                       // null = partial sums only, added by fp8_splitk_reduce_kernel
-  float* handoff;      // with tickets: [splits][T][N] partial sums in this launch's half of the context's
-                       // handoff buffer, which holds the empty pattern wherever this launch reads
-  uint4* restore;      // with tickets: the other half, whose first restore_n 16-byte words the previous
-  int64_t restore_n;   // launch wrote: every workgroup puts back the empty pattern over its share
-  const uint16_t* x;   // fused tile GEMV (block 128, few tokens): the BF16 input [T][K], quantized in the kernel
+  float* partial;      // split-K GEMM: [splits][T][N] FP32 partial sums (written instead of y)
+  const uint16_t* x;   // fused GEMV (few tokens): the BF16 input [T][K], quantized in the kernel
+  int ordered;         // GEMV: xq and xs as fp8_quant_ordered_kernel writes them, else [T][K] rows
   int64_t x_stride;    // activation elements per token: K, or groups x K when grouped
-  int x_group_rows;    // grouped activations (block-32 GEMV): weight rows [g R, (g + 1) R) multiply
+  int x_group_rows;    // grouped activations (block-32 GEMV, rows): weight rows [g R, (g + 1) R) multiply
                        // activation group g, codes at xq + tok x_stride + g K; 0 = one group
+  // gate/up pair (kPair): blob is W1 and blob2 W3, y and y3 (nullable) their BF16 outputs
+  const uint8_t* blob2;
+  uint16_t* y3;
+  uint16_t* din;         // [T][N] BF16: silu(W1 x) * (W3 x) [* route_w], clamped
+  float* swiglu_trace;   // [T][N][5], nullable
+  const float* route_w;  // [T] or null
+  float limit;
 };
 
-// Block-128 calls of up to kFusedMaxTokens tokens run on fp8_tile_gemv_kernel, which can quantize its own
-// activations into LDS rows of 128 codes + 16 bytes of padding; at 16 tokens the repeated quantization in
-// every workgroup costs more than the quantizer launch (measured).
+// Decode GEMV over 16-row MFMA tiles for up to 16 NT tokens. A workgroup of W waves owns M tile sets of TM
+// consecutive tiles over all of K: wave w takes set w % M and the (w / M)-th of W / M contiguous K parts, streams its
+// chunks (2 KB of weights per tile and chunk, non-temporal loads, each chunk's activation operands loaded once for its
+// TM tiles) through a register ring of row_ring chunks, and the K parts' partial tiles are added through LDS in
+// K-part order. No K range is shared between workgroups, so no partial sums leave the workgroup: no
+// handoff, no reduce launch.
+// Bound by the weight stream and, for several tokens, by the requests that the activations add to it: a chunk's codes
+// of 16 tokens as row pieces were 32 requests and their scales 16, beside 16 for a tile's weights, so a wave takes two
+// tiles where there are enough and the codes come in load order (fp8_quant_ordered_kernel). 16 tokens, us a call:
+// 7168 x 16384 32.4 -> 23.4, 24576 x 1536 14.3 -> 10.7, 2112 x 7168 13.4 -> 9.9 against 64-row groups with K split over
+// workgroups, and 44.8 -> 28.1 / 19.3 -> 12.5 / 16.4 -> 12.2 at 32 tokens, whose weights are read once (NT = 2).
+// Fused (few tokens): the M waves of a K part first quantize its chunks of the call's tokens (P passes of 4 blocks
+// of 128 values each) into the part's LDS rows with the quantizer launches' arithmetic, so the call needs none.
+// Pair: the two tiles of a set are the same 16 rows of W1 and W3, and the workgroup finishes with SwiGLU.
 constexpr int kFusedMaxTokens = 4;
-constexpr int kFusedRow = 144;
+constexpr int kFusedRow = 144;    // an LDS row: 128 codes + 16 bytes of padding
+constexpr int kTileQRows = 16;    // fused: at most 4 passes of 4 blocks per wave
 
-template <int kBlock>
-struct Fp8Chunk {
-  uint4 a[kTiles][2];
-  uint4 b0, b1;
-  uint32_t sw;   // block 32: scale word (byte t = tile t); block 128: FP32 bits of the weight block scale
-  uint32_t sx;   // block 32: 4 activation E8M0 codes of the chunk; block 128: FP32 bits of the act scale
+__host__ __device__ constexpr int row_ring(int TM) { return TM == 1 ? 4 : 3; }
+
+template <int TM, int NT>
+struct RowChunk {
+  uint4 a[TM][2];   // weights: a tile's two 1 KB halves of the chunk, 16 bytes per lane
+  uint32_t sw[2];   // block 32: the chunk's weight scale word (byte t = tile t of the row group); pair: W3's, too
+  uint4 b[NT][2];   // activation codes (unfused)
+  uint32_t sx[NT];  // unfused: block 32 the token's 4 E8M0 codes of the chunk, block 128 its FP32 scale's bits
 };
 
-// xsrow: this lane's token's activation scales (block 32: E8M0 bytes, block 128: FP32), chunk 0 first.
-template <int kBlock>
-__device__ __forceinline__ void fp8_load(Fp8Chunk<kBlock>& r, const Fp8Args& a, const uint8_t* wlane,
-                                         const uint8_t* slane, const float* swrow, const uint8_t* xrow,
-                                         const uint8_t* xsrow, int c, int q) {
-  // weights: non-temporal loads (each byte is read once per call); 48.8 against 53.0 us for the
-  // configuration-3 projections at T = 1 with plain loads (MI355X)
-#pragma unroll
-  for (int t = 0; t < kTiles; ++t) {
-    r.a[t][0] = ldg128_nt(wlane + (size_t)c * 8192 + t * 2048);
-    r.a[t][1] = ldg128_nt(wlane + (size_t)c * 8192 + t * 2048 + 1024);
-  }
-  r.b0 = ldg128(xrow + (size_t)c * 128 + 16 * q);
-  r.b1 = ldg128(xrow + (size_t)c * 128 + 64 + 16 * q);
-  if constexpr (kBlock == 32) {
-    r.sw = ldg32(slane + (size_t)c * 256);
-    r.sx = ldg32(xsrow + 4 * c);
-  } else {
-    r.sw = __float_as_uint(ldgf(swrow + c));
-    r.sx = __float_as_uint(ldgf(reinterpret_cast<const float*>(xsrow) + c));
-  }
-}
-
-template <int kBlock>
-__device__ __forceinline__ void fp8_mma(const Fp8Chunk<kBlock>& r, v4f (&acc)[kTiles], int q, uint32_t keep) {
-  const uint4 b0 = make_uint4(r.b0.x & keep, r.b0.y & keep, r.b0.z & keep, r.b0.w & keep);
-  const uint4 b1 = make_uint4(r.b1.x & keep, r.b1.y & keep, r.b1.z & keep, r.b1.w & keep);
-  if constexpr (kBlock == 32) {
-    const int sx = (int)((r.sx >> (8 * q)) & 0xFF);
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t)
-      acc[t] = mfma_fp8_fp8(r.a[t][0], r.a[t][1], b0, b1, acc[t], (int)((r.sw >> (8 * t)) & 0xFF), sx);
-  } else {
-    // the chunk's combined scale f32(sa * sw), then one fused multiply-add per output
-    const float s = __uint_as_float(r.sx) * __uint_as_float(r.sw);
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      const v4f d = mfma_fp8_fp8(r.a[t][0], r.a[t][1], b0, b1, v4f{0.f, 0.f, 0.f, 0.f}, 127, 127);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[i], s, acc[t][i]);
-    }
-  }
-}
-
-// grid (N / 64, ceil(T / 16), splits), 256 threads: 64 weight rows x 16 tokens x one K range per
-// workgroup. Wave w streams its quarter of the workgroup's K chunks (P = 2 chunks of 8 KB in flight), the
-// quarters are summed through LDS in wave order, then wave t writes tile t: BF16 (and the FP32 trace)
-// when K is not split, else its FP32 partial sums. With K split and a.tickets set, the last workgroup of
-// the (row group, token tile) to arrive adds the partial sums in split order (fp8_splitk_reduce_kernel's
-// arithmetic) and writes the outputs; without tickets fp8_splitk_reduce_kernel does it.
-template <int kBlock>
-__global__ __launch_bounds__(256) void fp8_gemv_kernel(Fp8Args a) {
-  constexpr int P = 2;
-  const int g = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q = lane >> 4, n = lane & 15;
-  const int tok = blockIdx.y * kTok + n;
-  const bool live = tok < a.T;
-  const int rtok = live ? tok : a.T - 1;
-  const int C = a.K / 128;
-  const Fp8Blob off = fp8_blob(a.N, a.K, kBlock);
-  const uint8_t* wlane = a.blob + (size_t)g * C * 8192 + 16 * lane;
-  const uint8_t* slane = a.blob + off.scales + (size_t)g * C * 256 + 4 * lane;
-  const float* swrow = reinterpret_cast<const float*>(a.blob + off.scales) + (size_t)((64 * g) / 128) * C;
-  // grouped activations: the row group's 64 rows lie in one activation group (x_group_rows % 64 == 0)
-  const int xgroup = a.x_group_rows ? (64 * g) / a.x_group_rows : 0;
-  const uint8_t* xrow = a.xq + (size_t)rtok * a.x_stride + (size_t)xgroup * a.K;
-  const uint8_t* xsrow =
-      kBlock == 32 ? (const uint8_t*)a.xs + (size_t)rtok * (a.x_stride / 32) + (size_t)xgroup * (a.K / 32)
-                   : reinterpret_cast<const uint8_t*>((const float*)a.xs + (size_t)rtok * (a.K / 128));
-  if (a.restore_n) {
-    // this workgroup's share of the other handoff half (plain stores: the kernel boundary publishes them
-    // to the launch that uses that half next)
-    const int64_t wg = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    const int64_t wgs = (int64_t)gridDim.x * gridDim.y * gridDim.z;
-    const int64_t per = (a.restore_n + wgs - 1) / wgs;
-    const uint4 empty = make_uint4(mxd::kHandoffEmpty, mxd::kHandoffEmpty, mxd::kHandoffEmpty, mxd::kHandoffEmpty);
-    for (int64_t i = wg * per + tid; i < min((wg + 1) * per, a.restore_n); i += 256) a.restore[i] = empty;
-  }
-  v4f acc[kTiles];
-#pragma unroll
-  for (int t = 0; t < kTiles; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int z = blockIdx.z, S = gridDim.z;
-  const int cb = (C * z) / S, cw = (C * (z + 1)) / S - cb;   // this workgroup's chunk range
-  const int c0 = cb + (cw * wave) / 4;
-  const int cn = cb + (cw * (wave + 1)) / 4 - c0;
-  const uint32_t keep = live ? 0xFFFFFFFFu : 0u;
-  Fp8Chunk<kBlock> buf[P];
-  if (cn > 0) {
-#pragma unroll
-    for (int j = 0; j < P; ++j) fp8_load<kBlock>(buf[j], a, wlane, slane, swrow, xrow, xsrow, c0 + min(j, cn - 1), q);
-    int i = 0;
-    for (; i + P < cn; i += P) {
-#pragma unroll
-      for (int j = 0; j < P; ++j) {
-        fp8_mma<kBlock>(buf[j], acc, q, keep);
-        fp8_load<kBlock>(buf[j], a, wlane, slane, swrow, xrow, xsrow, c0 + min(i + j + P, cn - 1), q);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < P; ++j) fp8_mma<kBlock>(buf[j], acc, q, i + j < cn ? keep : 0u);
-  }
-  __shared__ float red[4][kTiles][64][4];
-#pragma unroll
-  for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][t][lane][i] = acc[t][i];
-  __syncthreads();
-  float out[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    out[i] = ((red[0][wave][lane][i] + red[1][wave][lane][i]) + red[2][wave][lane][i]) + red[3][wave][lane][i];
-  const size_t o = (size_t)tok * a.N + 64 * g + 16 * wave + 4 * q;
-  if (S > 1) {
-    float* part = a.partial + (size_t)z * a.T * a.N + o;
-    if (!a.tickets) {
-      if (live) *reinterpret_cast<float4*>(part) = make_float4(out[0], out[1], out[2], out[3]);
-      return;
-    }
-    // The partial sums go to this launch's half of the context's handoff buffer (a.handoff, [S][T][N] FP32),
-    // which holds the kHandoffEmpty pattern wherever this launch reads (the launch before restored it):
-    // each pair of sums is published as one 64-bit agent-scope atomic, a relaxed atomic ticket per tile
-    // elects the last of the S arrivals, and that workgroup reads every split's pairs, re-reading any
-    // location that still holds the empty pattern until the published pair is visible, and adds them in
-    // split order. In a launch a location only ever holds the empty pattern or this launch's pair, so
-    // correctness rests on per-location coherence of the atomics (and the kernel boundaries between
-    // launches) -- not on an order between different locations, which would need agent-scope fences: each
-    // release fence writes back the XCD's whole L2, tens of microseconds over a launch. The stores have
-    // completed before the ticket is taken (s_waitcnt 0, then the barrier), so the first read normally finds
-    // them; the re-reads are bounded, and a pair still missing at the bound becomes NaN instead of a hang.
-    const size_t stride = (size_t)a.T * a.N;
-    float* hand = a.handoff + o;
-    if (live) {
-      mxd::store_device(hand + (size_t)z * stride, out[0], out[1]);
-      mxd::store_device(hand + (size_t)z * stride + 2, out[2], out[3]);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __shared__ uint32_t arrived;
-    __syncthreads();
-    uint32_t* ticket = a.tickets + (size_t)blockIdx.y * gridDim.x + g;
-    if (tid == 0) arrived = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (arrived != (uint32_t)(S - 1)) return;
-    if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (!live) return;
-    float2 p[16][2];
-#pragma unroll
-    for (int zz = 0; zz < 16; ++zz)
-      if (zz < S) {
-        p[zz][0] = mxd::load_device(hand + (size_t)zz * stride);
-        p[zz][1] = mxd::load_device(hand + (size_t)zz * stride + 2);
-      }
-    // one check over every pair first; the re-reads are the rare path
-    bool missing = false;
-#pragma unroll
-    for (int zz = 0; zz < 16; ++zz)
-      if (zz < S)
-        missing |= (int)(__float_as_uint(p[zz][0].x) == mxd::kHandoffEmpty) |
-                    (int)(__float_as_uint(p[zz][1].x) == mxd::kHandoffEmpty);
-    if (missing) {
-#pragma unroll
-      for (int zz = 0; zz < 16; ++zz)
-        if (zz < S) {   // unrolled: p stays in registers
-          p[zz][0] = mxd::await_pair(p[zz][0], hand + (size_t)zz * stride);
-          p[zz][1] = mxd::await_pair(p[zz][1], hand + (size_t)zz * stride + 2);
-        }
-    }
-    float4 t = make_float4(p[0][0].x, p[0][0].y, p[0][1].x, p[0][1].y);
-#pragma unroll
-    for (int zz = 1; zz < 16; ++zz)
-      if (zz < S) {
-        t.x = t.x + p[zz][0].x;
-        t.y = t.y + p[zz][0].y;
-        t.z = t.z + p[zz][1].x;
-        t.w = t.w + p[zz][1].y;
-      }
-    out[0] = t.x;
-    out[1] = t.y;
-    out[2] = t.z;
-    out[3] = t.w;
-  }
-  if (live) {
-    uint2 packed;
-    packed.x = mx::bf16_bits(out[0]) | (mx::bf16_bits(out[1]) << 16);
-    packed.y = mx::bf16_bits(out[2]) | (mx::bf16_bits(out[3]) << 16);
-    *reinterpret_cast<uint2*>(a.y + o) = packed;
-    if (a.trace) *reinterpret_cast<float4*>(a.trace + o) = make_float4(out[0], out[1], out[2], out[3]);
-  }
-}
-
-// Block-128 decode GEMV over 16-row tiles. A workgroup of W waves owns M consecutive 16-row MFMA tiles
-// (one token tile) over all of K: wave w takes tile w % M and the (w / M)-th of W / M contiguous K parts,
-// streams its chunks through a register ring of kTileRing chunks (2 KB of weights per chunk, non-temporal
-// loads) into one FP32 16 x 16 partial tile, acc = fma(d, f32(sa sw), acc) in chunk order, and each tile's
-// W / M partial tiles are added through LDS in K-part order. No K range is shared between workgroups, so no
-// partial sums leave the workgroup (no handoff, no reduce launch); the host picks W and M so that the launch
-// has a few thousand waves in a few hundred workgroups.
-// Fused (few tokens): the M waves of a K part first quantize its chunks of the call's tokens (P passes of 4
-// blocks of 128 each) into the part's LDS rows with act_quant128_v8_kernel's arithmetic, so the call needs no
-// quantizer launch.
-constexpr int kTileRing = 4;
-constexpr int kTileQRows = 16;   // fused: at most 4 passes of 4 blocks per wave
-
-struct TileChunk {
-  uint4 a0, a1;   // weights: the tile's two 1 KB halves of the chunk, 16 bytes per lane
-  uint4 b0, b1;   // activation codes (unfused)
-  float sx;       // activation scale (unfused)
+// Where a lane reads its operands; chunk c's are at fixed strides from these.
+template <int TM, int NT>
+struct RowSource {
+  const uint8_t* w[TM];    // tile t's halves of chunk c at + 8192 c and + 8192 c + 1024
+  const uint8_t* sw[TM];   // block 32: the scale words at + 256 c (one word serves the tiles of one row group)
+  const uint8_t* x[NT];    // the lane's codes: 16 bytes at + x_chunk c and x_half further
+  const uint8_t* xs[NT];   // and its token's scales, chunk c's 4 bytes at + xs_chunk c
+  int x_chunk, x_half, xs_chunk;
 };
 
-template <bool kFused>
-__device__ __forceinline__ void tile_load(TileChunk& r, const uint8_t* wlane, const uint8_t* xrow,
-                                          const float* xsrow, int c, int q) {
-  r.a0 = ldg128_nt(wlane + (size_t)c * 8192);
-  r.a1 = ldg128_nt(wlane + (size_t)c * 8192 + 1024);
+template <int kBlock, bool kFused, int TM, int NT, bool kPair>
+__device__ __forceinline__ void row_load(RowChunk<TM, NT>& r, const RowSource<TM, NT>& s, int c) {
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    r.a[t][0] = ldg128_nt(s.w[t] + (size_t)c * 8192);
+    r.a[t][1] = ldg128_nt(s.w[t] + (size_t)c * 8192 + 1024);
+  }
+  if constexpr (kBlock == 32) {
+    r.sw[0] = ldg32(s.sw[0] + (size_t)c * 256);
+    if constexpr (kPair) r.sw[1] = ldg32(s.sw[TM - 1] + (size_t)c * 256);
+  }
   if constexpr (!kFused) {
-    r.b0 = ldg128(xrow + (size_t)c * 128 + 16 * q);
-    r.b1 = ldg128(xrow + (size_t)c * 128 + 64 + 16 * q);
-    r.sx = ldgf(xsrow + c);
-  }
-}
-
-// sw: the chunk's weight block scale; row / qs: fused, this lane's token's LDS row and scale for the chunk,
-// unused otherwise
-template <bool kFused>
-__device__ __forceinline__ void tile_mma(const TileChunk& r, v4f& acc, int q, uint32_t keep, float sw,
-                                         const uint8_t* row, const float* qs) {
-  uint4 b0 = r.b0, b1 = r.b1;
-  float sx = r.sx;
-  if constexpr (kFused) {
-    b0 = *reinterpret_cast<const uint4*>(row + 16 * q);
-    b1 = *reinterpret_cast<const uint4*>(row + 64 + 16 * q);
-    sx = *qs;
-  }
-  b0 = make_uint4(b0.x & keep, b0.y & keep, b0.z & keep, b0.w & keep);
-  b1 = make_uint4(b1.x & keep, b1.y & keep, b1.z & keep, b1.w & keep);
-  const float s = sx * sw;
-  const v4f d = mfma_fp8_fp8(r.a0, r.a1, b0, b1, v4f{0.f, 0.f, 0.f, 0.f}, 127, 127);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = fmaf(d[i], s, acc[i]);
+    for (int u = 0; u < NT; ++u) {
+      const uint8_t* x = s.x[u] + (size_t)c * s.x_chunk;
+      r.b[u][0] = ldg128(x);
+      r.b[u][1] = ldg128(x + s.x_half);
+      r.sx[u] = ldg32(s.xs[u] + (size_t)c * s.xs_chunk);
+    }
+  }
 }
 
 __device__ __forceinline__ float chunk_scale(float swl, int i) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(swl), i));
 }
 
-// grid (N / 16 / M, ceil(T / 16)), 64 W threads.
-template <bool kFused, int W, int M, int P>
-__global__ __launch_bounds__(64 * W) void fp8_tile_gemv_kernel(Fp8Args a) {
-  static_assert(W % M == 0 && 4 * P * M <= kTileQRows, "tile GEMV shape");
-  constexpr int KP = W / M;
+// One chunk into the accumulators. tsel: the first tile's index in its row group (its scale byte); swf: block 128,
+// the chunk's weight block scale; keep[u]: all ones where this lane's token of tile u is in use, else zero; row / qs:
+// fused, this lane's token's LDS row and scale word.
+template <int kBlock, bool kFused, int TM, int NT, bool kPair>
+__device__ __forceinline__ void row_mma(const RowChunk<TM, NT>& r, v4f (&acc)[NT][TM], int q,
+                                        const uint32_t (&keep)[NT], int tsel, float swf, const uint8_t* row,
+                                        const uint32_t* qs) {
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    uint4 b0 = r.b[u][0], b1 = r.b[u][1];
+    uint32_t sx = r.sx[u];
+    if constexpr (kFused) {
+      b0 = *reinterpret_cast<const uint4*>(row + 16 * q);
+      b1 = *reinterpret_cast<const uint4*>(row + 64 + 16 * q);
+      sx = *qs;
+    }
+    b0 = make_uint4(b0.x & keep[u], b0.y & keep[u], b0.z & keep[u], b0.w & keep[u]);
+    b1 = make_uint4(b1.x & keep[u], b1.y & keep[u], b1.z & keep[u], b1.w & keep[u]);
+    if constexpr (kBlock == 32) {
+      const int xb = (int)((sx >> (8 * q)) & 0xFF);
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+        const int ws = (int)((r.sw[kPair && t ? 1 : 0] >> (8 * (kPair ? tsel : tsel + t))) & 0xFF);
+        acc[u][t] = mfma_fp8_fp8(r.a[t][0], r.a[t][1], b0, b1, acc[u][t], ws, xb);
+      }
+    } else {
+      const float s = __uint_as_float(sx) * swf;
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+        const v4f d = mfma_fp8_fp8(r.a[t][0], r.a[t][1], b0, b1, v4f{0.f, 0.f, 0.f, 0.f}, 127, 127);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[u][t][i] = fmaf(d[i], s, acc[u][t][i]);
+      }
+    }
+  }
+}
+
+// grid (ceil(tile sets / M), ceil(T / (16 NT))), 64 W threads.
+template <int kBlock, bool kFused, int W, int M, int TM, int NT, int P, bool kPair>
+__global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
+  static_assert(W % M == 0 && 4 * P * M <= kTileQRows && M * TM * NT <= W && (NT == 1 || !kFused) &&
+                    (!kPair || (TM == 2 && NT == 1 && M == 1 && kBlock == 32)),
+                "row GEMV shape");
+  constexpr int KP = W / M, R = row_ring(TM);
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tile = blockIdx.x * M + w % M, kp = w / M;
+  const int kp = w / M, sets = kPair ? a.N / 16 : a.N / 16 / TM;
+  const int set_raw = blockIdx.x * M + w % M, set = min(set_raw, sets - 1);   // a set past the last repeats it
+  const int tile = kPair ? set : set * TM;
   const int q = lane >> 4, nn = lane & 15;
-  const int tok0 = blockIdx.y * kTok, tok = tok0 + nn;
-  const int ntok = min(kTok, a.T - tok0);
-  const bool live = nn < ntok;
-  const int rtok = live ? tok : a.T - 1;
-  const int C = a.K / 128;
-  const Fp8Blob off = fp8_blob(a.N, a.K, 128);
-  // tile t of row group g: chunk c's halves at (g C + c) 8192 + 2048 t + {0, 1024}
-  const uint8_t* wlane = a.blob + (size_t)(tile >> 2) * C * 8192 + (tile & 3) * 2048 + 16 * lane;
+  const int tok0 = blockIdx.y * (kTok * NT);
+  const int ntok = min(kTok * NT, a.T - tok0);   // the workgroup's tokens; token tile u holds tok0 + 16 u ..
+  const int C = a.K / 128, g = tile >> 2;
+  const Fp8Blob off = fp8_blob(a.N, a.K, kBlock);
   const float* swrow = reinterpret_cast<const float*>(a.blob + off.scales) + (size_t)(tile >> 3) * C;
-  const uint8_t* xrow = a.xq + (size_t)rtok * a.K;
-  const float* xsrow = reinterpret_cast<const float*>(a.xs) + (size_t)rtok * C;
+  // grouped activations: a set's rows lie in one activation group (x_group_rows % 64 == 0)
+  const int xgroup = a.x_group_rows ? (16 * tile) / a.x_group_rows : 0;
+  RowSource<TM, NT> src;
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    const uint8_t* blob = kPair && t ? a.blob2 : a.blob;
+    const int tl = kPair ? tile : tile + t;
+    src.w[t] = blob + (size_t)g * C * 8192 + (tl & 3) * 2048 + 16 * lane;
+    src.sw[t] = blob + off.scales + (size_t)g * C * 256 + 4 * lane;
+  }
+  uint32_t keep[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    // idle columns read the last token's bytes
+    const int local = min(16 * u + nn, ntok - 1);
+    keep[u] = 16 * u + nn < ntok ? 0xFFFFFFFFu : 0u;
+    if (a.ordered) {
+      const size_t tt = (size_t)((tok0 + local) >> 4) * C;
+      src.x[u] = a.xq + tt * 2048 + 16 * (16 * q + (local & 15));
+      src.xs[u] = (const uint8_t*)a.xs + tt * 64 + 4 * (local & 15);
+    } else {
+      const size_t at = (size_t)(tok0 + local) * a.x_stride + (size_t)xgroup * a.K;
+      src.x[u] = a.xq + at + 16 * q;
+      src.xs[u] = (const uint8_t*)a.xs + at / 32;
+    }
+  }
+  src.x_chunk = a.ordered ? 2048 : 128;
+  src.x_half = a.ordered ? 1024 : 64;
+  src.xs_chunk = a.ordered ? 64 : 4;
   const int c0 = (C * kp) / KP, n = (C * (kp + 1)) / KP - c0;
   // fused: K part kp's rows, block b = i ntok + token (chunk c0 + i), 128 codes + 16 bytes of padding each,
   // quantized by the part's M waves together (wave w % M takes blocks 4 P (w % M) + 0 .. 4 P - 1), then one
   // spare row per wave that takes the stores of lanes past the part's blocks (no branch around the math:
-  // branches would make the compiler wait for the weight loads before quantizing)
+  // branches would make the compiler wait for the weight loads before quantizing). qsc: a row's scales, block 32
+  // four E8M0 bytes, block 128 one FP32
   constexpr int kPartRows = 4 * P * M;
   __shared__ __attribute__((aligned(16))) uint8_t qx[kFused ? (KP * kPartRows + W) * kFusedRow : 16];
-  __shared__ float qsc[kFused ? KP * kPartRows + W : 1];
+  __shared__ uint32_t qsc[kFused ? KP * kPartRows + W : 1];
   const int sub = lane & 15, grp = lane >> 4;
   const int nb = n * ntok, nl = max(n - 1, 0), b0 = 4 * P * (w % M);
   uint4 xv[kFused ? P : 1];
@@ -464,31 +381,33 @@ __global__ __launch_bounds__(64 * W) void fp8_tile_gemv_kernel(Fp8Args a) {
   // the activation loads first, then the ring, then the quantization: loads return in order, so quantizing
   // waits for the activations alone (scheduling barriers keep the compiler from interleaving the three)
   __builtin_amdgcn_sched_barrier(0);
-  // the wave's weight block scales, lane i holding chunk c0 + i's (at most 64 chunks a wave, checked on the
-  // host); each chunk's is read out with v_readlane into a scalar register
-  const float swl = ldgf(swrow + c0 + min(lane, nl));
-  TileChunk buf[kTileRing];
+  // block 128: the wave's weight block scales, lane i holding chunk c0 + sw0 + i's; each chunk's is read out with
+  // v_readlane into a scalar register
+  int sw0 = 0;
+  float swl = 0.f;
+  if constexpr (kBlock == 128) swl = ldgf(swrow + c0 + min(lane, nl));
+  auto next_scales = [&](int i) {
+    sw0 = i;
+    swl = ldgf(swrow + c0 + min(sw0 + lane, nl));
+    asm volatile("" : "+v"(swl));   // waited for here, not where the paths with and without this load meet
+  };
+  RowChunk<TM, NT> buf[R];
 #pragma unroll
-  for (int j = 0; j < kTileRing; ++j) tile_load<kFused>(buf[j], wlane, xrow, xsrow, c0 + min(j, nl), q);
+  for (int j = 0; j < R; ++j) row_load<kBlock, kFused, TM, NT, kPair>(buf[j], src, c0 + min(j, nl));
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (kFused) {
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int b = b0 + 4 * p + grp;
-      const uint32_t wd[4] = {xv[p].x, xv[p].y, xv[p].z, xv[p].w};
-      float v[8];
-      float amax = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = mx::bf16_value(wd[i] & 0xFFFFu);
-        v[2 * i + 1] = mx::bf16_value(wd[i] >> 16);
-        amax = fmaxf(amax, fmaxf(fabsf(v[2 * i]), fabsf(v[2 * i + 1])));
-      }
-      amax = mxd::row16_max(amax);
-      const float sc = mx::act128_scale(amax);
       const int row = b < nb ? kp * kPartRows + b : KP * kPartRows + w;
-      *reinterpret_cast<uint2*>(qx + row * kFusedRow + 8 * sub) = act128_codes8(v, sc);
-      if (sub == 0) qsc[row] = sc;
+      uint32_t scale;
+      const uint2 codes = quantize8<kBlock>(xv[p], scale);
+      if constexpr (kBlock == 32) {
+        if ((sub & 3) == 0) reinterpret_cast<uint8_t*>(qsc + row)[sub >> 2] = (uint8_t)scale;
+      } else {
+        if (sub == 0) qsc[row] = scale;
+      }
+      *reinterpret_cast<uint2*>(qx + row * kFusedRow + 8 * sub) = codes;
     }
     if constexpr (M == 1) {
       // the rows are this wave's own: its LDS writes complete before its reads (no workgroup barrier)
@@ -497,56 +416,94 @@ __global__ __launch_bounds__(64 * W) void fp8_tile_gemv_kernel(Fp8Args a) {
       mxd::lds_barrier();   // the part's rows come from M waves; LDS only, the weight loads stay in flight
     }
   }
-  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-  const uint32_t keep = live ? 0xFFFFFFFFu : 0u;
+  v4f acc[NT][TM];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int t = 0; t < TM; ++t) acc[u][t] = v4f{0.f, 0.f, 0.f, 0.f};
   const int qtok = kFused ? min(nn, ntok - 1) : 0;
   const uint8_t* qrow = qx + (kp * kPartRows + qtok) * kFusedRow;
-  const float* qs = qsc + kp * kPartRows + qtok;
+  const uint32_t* qs = qsc + kp * kPartRows + qtok;
   int i = 0;
-  for (; i + kTileRing < n; i += kTileRing) {
+  for (; i + R < n; i += R) {
+    if constexpr (kBlock == 128)
+      if (i + R > sw0 + 64) next_scales(i);
 #pragma unroll
-    for (int j = 0; j < kTileRing; ++j) {
-      // a ring: chunk i + j is multiplied, then its slot is refilled with chunk i + j + kTileRing before the
-      // next chunk is waited for (the barrier keeps the compiler from batching the loads after all four)
-      tile_mma<kFused>(buf[j], acc, q, keep, chunk_scale(swl, i + j), qrow + (i + j) * ntok * kFusedRow,
-                       qs + (i + j) * ntok);
-      tile_load<kFused>(buf[j], wlane, xrow, xsrow, c0 + min(i + j + kTileRing, nl), q);
+    for (int j = 0; j < R; ++j) {
+      // a ring: chunk i + j is multiplied, then its slot is refilled with chunk i + j + R before the next chunk is
+      // waited for (the barrier keeps the compiler from batching the loads after all of them)
+      row_mma<kBlock, kFused, TM, NT, kPair>(buf[j], acc, q, keep, tile & 3,
+                                             kBlock == 128 ? chunk_scale(swl, i + j - sw0) : 0.f,
+                                             qrow + (i + j) * ntok * kFusedRow, qs + (i + j) * ntok);
+      row_load<kBlock, kFused, TM, NT, kPair>(buf[j], src, c0 + min(i + j + R, nl));
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if constexpr (kBlock == 128)
+    if (i + R > sw0 + 64) next_scales(i);
 #pragma unroll
-  for (int j = 0; j < kTileRing; ++j) {
-    const int ij = min(i + j, nl);
-    tile_mma<kFused>(buf[j], acc, q, i + j < n ? keep : 0u, chunk_scale(swl, ij), qrow + ij * ntok * kFusedRow,
-                     qs + ij * ntok);
-  }
-  __shared__ float4 red[W][64];
-  red[w][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  for (int j = 0; j < R; ++j)
+    if (i + j < n)
+      row_mma<kBlock, kFused, TM, NT, kPair>(buf[j], acc, q, keep, tile & 3,
+                                             kBlock == 128 ? chunk_scale(swl, i + j - sw0) : 0.f,
+                                             qrow + (i + j) * ntok * kFusedRow, qs + (i + j) * ntok);
+  __shared__ float4 red[W][TM * NT][64];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+      red[w][TM * u + t][lane] = make_float4(acc[u][t][0], acc[u][t][1], acc[u][t][2], acc[u][t][3]);
   __syncthreads();
-  if (w >= M || !live) return;
-  // wave w < M finishes tile w: K-part order, over the parts that own chunks (KP > C leaves some without)
-  float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-  bool first = true;
+  // wave w < M TM NT finishes tile (w / M) % TM of set w % M for token tile w / (M TM): K-part order, over the parts
+  // that own chunks (KP > C leaves some without)
+  float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int ft = w / M;
+  if (w < M * TM * NT) {
+    bool first = true;
 #pragma unroll
-  for (int v = 0; v < KP; ++v) {
-    if ((C * (v + 1)) / KP == (C * v) / KP) continue;
-    const float4 r = red[w + M * v][lane];
-    if (first) {
-      t = r;
-      first = false;
-    } else {
-      t.x = t.x + r.x;
-      t.y = t.y + r.y;
-      t.z = t.z + r.z;
-      t.w = t.w + r.w;
+    for (int v = 0; v < KP; ++v) {
+      if ((C * (v + 1)) / KP == (C * v) / KP) continue;
+      const float4 r = red[w % M + M * v][ft][lane];
+      if (first) {
+        o4 = r;
+        first = false;
+      } else {
+        o4.x = o4.x + r.x;
+        o4.y = o4.y + r.y;
+        o4.z = o4.z + r.z;
+        o4.w = o4.w + r.w;
+      }
     }
   }
-  const size_t o = (size_t)tok * a.N + 16 * tile + 4 * q;
+  if constexpr (kPair) {
+    // element (token, row) per thread: gate and up of it from LDS
+    __shared__ float pair[2][kTok][16 + 1];
+    if (w < 2 && nn < ntok) {
+      const float v[4] = {o4.x, o4.y, o4.z, o4.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pair[w][nn][4 * q + e] = v[e];
+    }
+    __syncthreads();
+    for (int p = tid; p < 16 * ntok; p += 64 * W) {
+      const int pt = p >> 4, row = p & 15;
+      const size_t o = (size_t)(tok0 + pt) * a.N + 16 * tile + row;
+      const uint32_t b1 = mx::bf16_bits(pair[0][pt][row]), b3 = mx::bf16_bits(pair[1][pt][row]);
+      const float v = mxd::swiglu_element(b1, b3, a.limit, a.route_w != nullptr, a.route_w ? a.route_w[tok0 + pt] : 1.f,
+                                          a.swiglu_trace ? a.swiglu_trace + o * 5 : nullptr);
+      a.din[o] = (uint16_t)mx::bf16_bits(v);
+      if (a.y) a.y[o] = (uint16_t)b1;
+      if (a.y3) a.y3[o] = (uint16_t)b3;
+    }
+    return;
+  }
+  const int local = 16 * (ft / TM) + nn;
+  if (w >= M * TM * NT || local >= ntok || set_raw >= sets) return;
+  const size_t o = (size_t)(tok0 + local) * a.N + 16 * (tile + ft % TM) + 4 * q;
   uint2 packed;
-  packed.x = mx::bf16_bits(t.x) | (mx::bf16_bits(t.y) << 16);
-  packed.y = mx::bf16_bits(t.z) | (mx::bf16_bits(t.w) << 16);
+  packed.x = mx::bf16_bits(o4.x) | (mx::bf16_bits(o4.y) << 16);
+  packed.y = mx::bf16_bits(o4.z) | (mx::bf16_bits(o4.w) << 16);
   *reinterpret_cast<uint2*>(a.y + o) = packed;
-  if (a.trace) *reinterpret_cast<float4*>(a.trace + o) = t;
+  if (a.trace) *reinterpret_cast<float4*>(a.trace + o) = o4;
 }
 
 // Split-K epilogue: y = BF16(sum over splits in order), 4 outputs per thread.
@@ -754,96 +711,108 @@ int check_fp8_shape(int N, int K, int block, const char* who) {
   return MX_OK;
 }
 
-// K splits. Decode GEMV: see below. GEMM: only when the rows and tokens alone give fewer workgroups than
-// half the CUs (the partial sums cost a write and a read of splits x T x N floats and a reduce launch), then
-// about 512, every split keeping 8 chunks. 2112 x 7168 at T = 2048 (144 workgroups) ran 97 us per call
-// unsplit against 110 us with 4 splits (MI355X, quantizer included).
+// K splits of the GEMM: only when the rows and tokens alone give fewer workgroups than half the CUs (the partial
+// sums cost a write and a read of splits x T x N floats and a reduce launch), then about 512, every split keeping 8
+// chunks. 2112 x 7168 at T = 2048 (144 workgroups) ran 97 us per call unsplit against 110 us with 4 splits (MI355X,
+// quantizer included).
 int fp8_splits(int N, int K, int T) {
-  if (T > kGemvMaxTokens) {
-    const int base_wgs = ((N / 64 + 3) / 4) * ((T + kGemmTok - 1) / kGemmTok);
-    if (base_wgs >= 128) return 1;
-    return std::max(1, std::min({8, (K / 128) / 8, (512 + base_wgs - 1) / base_wgs}));
-  }
-  // Split-K GEMV: up to kFusedMaxTokens tokens every workgroup takes up to 16 chunks of its row group, else
-  // about 8; at most 16 splits. Fewer, longer workgroups measured faster than a fixed workgroup count on
-  // MI355X (us per call, T = 1 / 16): 2112 x 7168 7 splits 11.3 / 13.1 against 14 splits (the former
-  // ~512-workgroup rule) 12.5 / 16.9; 7168 x 16384 16 splits 28.9 / 33.8 against 5 splits 30.1 / 33.3. At T =
-  // 1 with non-temporal weight loads: 24576 x 1536 unsplit 10.3 us against 12.5 us with 2 splits (no split-K
-  // handoff); 2112 x 7168 4 splits 10.4 us, 7168 x 16384 8 splits 26.6 us, both as with 7 and 16. (Block-128
-  // calls of up to 4 tokens now run on the tile GEMV, which splits K only within a workgroup.)
-  const int chunks = K / 128;
-  const int s = T <= kFusedMaxTokens ? (chunks + 15) / 16 : chunks / 8;
-  return std::max(1, std::min(16, s));
+  if (T <= kGemvMaxTokens) return 1;
+  const int base_wgs = ((N / 64 + 3) / 4) * ((T + kGemmTok - 1) / kGemmTok);
+  if (base_wgs >= 128) return 1;
+  return std::max(1, std::min({8, (K / 128) / 8, (512 + base_wgs - 1) / base_wgs}));
 }
 
-// Shape of the block-128 decode GEMV (fp8_tile_gemv_kernel): W waves and M tiles per workgroup. Many tiles
-// (q_b's 1536): 2 tiles of 4 K parts; few tiles (q_kv_a's 132): 8 K parts of one tile; otherwise (o's 448)
-// 2 tiles of 8 K parts. Measured on MI355X at T = 1 (us per call, weights rotated): q_b 7.7-8.6 with 2 x 4
-// against 9.6-10.2 with 4 tiles x 4 parts, 10.0 with 4 x 2 and 11.8-12.1 with 2 x 8; q_kv_a 6.6-6.7 with
-// 1 x 8 against 6.9-7.0 with 1 x 16; o 21.1-21.4 with 2 x 8 against 22.0-22.5 with 1 x 8 and 22.8 with
-// 1 x 16. A 6-chunk ring left o unchanged and slowed q_kv_a.
-struct TileShape {
-  int W, M;
+// Shape of the decode GEMV: W waves a workgroup, M tile sets of TM tiles.
+struct RowShape {
+  int W, M, TM;
+  int parts() const { return W / M; }
 };
 
-TileShape fp8_tile_shape(int N, int T) {
-  const int tiles = (N / 16) * ((T + kTok - 1) / kTok);
-  if (tiles >= 1024) return {8, 2};
-  if (tiles * 16 <= 4096) return {8, 1};
-  return {16, 2};
-}
+// Gate/up of the FP8 expert. The 5120 x 2304 expert (two or four launches), us at 1 / 4 / 16 tokens: 13.7 / 17.8 / 20.4
+// with 8 waves, 14.7 / 17.8 / 21.2 with 16, 14.1 / 18.2 / 20.0 with 4; 31.6 / 33.0 / 34.7 as six launches (quantizer,
+// W1, W3, SwiGLU, quantizer, W2). Two launches of about 6 us for 35 MB: their ramps and drains bound it now.
+constexpr RowShape kPairShape{8, 1, 2};
 
-// Whether fp8_tile_gemv_kernel takes the call: every wave's chunks within the 64 lanes that hold their weight
-// scales (K up to 64 x 128 x the K parts).
-bool fp8_tile_ok(int N, int K, int T) {
-  const TileShape sh = fp8_tile_shape(N, T);
-  const int kp = sh.W / sh.M;
-  return (K / 128 + kp - 1) / kp <= 64;
+RowShape fp8_row_shape(int N, int K, int T) {
+  // us per call (quantizer launch included where there is one), weights rotated, W x M x TM:
+  // * up to 256 tiles: one tile a workgroup, 4 K parts, or 8 where one or two tokens leave the waves little else to do
+  //   and the parts stay 7 chunks long. 2112 x 7168: 4 parts 6.6 / 8.8 / 9.9 at 1 / 8 / 16 tokens, 8 parts 5.8 / 9.1 /
+  //   10.1, 16 parts 6.5 / 9.7 / 10.7; 1280 x 5120: 4 parts 5.6 / 7.7 / 8.4, 8 parts 5.8 / 8.7 / 9.5.
+  // * from 1024 tiles: two tiles a wave, 4 K parts; two sets a workgroup where 3 or 4 tokens are quantized in it (the
+  //   two waves of a part share that). 24576 x 1536: 4 x 1 x 2 8.0 / 9.3 / 10.3 / 10.7 at 1 / 4 / 8 / 16 tokens, 8 x 2 x
+  //   2 8.4 / 9.0 / 11.1 / 11.5, one tile a wave (8 x 2 x 1) 8.3 / 9.2 / 11.9 / 12.1.
+  // * between: few tokens, two tiles of 8 K parts (4 where the parts would be short); else two tiles a wave, so that
+  //   each activation operand is loaded for two products. 7168 x 16384: 16 x 2 x 1 20.4 / 22.7 / 22.7 / 24.9 at 1 / 4 / 8
+  //   / 16 tokens, 4 x 1 x 2 22.3 / 22.5 / 22.4 / 23.4; 5120 x 2304: 8 x 2 x 1 5.0 / 7.9 / 8.0 / 8.5, 16 x 2 x 1 6.1 / 6.6 /
+  //   8.7 / 9.0, 4 x 1 x 2 5.1 / 7.6 / 7.7 / 8.2.
+  const int tiles = N / 16, C = K / 128;
+  if (tiles <= 256) return {T <= 2 && C >= 56 ? 8 : 4, 1, 1};
+  if (tiles >= 1024) return T == 3 || T == 4 ? RowShape{8, 2, 2} : RowShape{4, 1, 2};
+  if (T <= 2 && C < 64) return {8, 2, 1};
+  if (T <= 4) return {16, 2, 1};
+  return {4, 1, 2};
 }
 
 // Fused quantization passes (4 blocks of 128 each per wave) for a K part's chunks x the tokens, shared by the
 // part's M waves: 1, 2 or 4, or 0 when they exceed the part's LDS rows (the call then quantizes in its own
 // launch).
-int fp8_tile_passes(int N, int K, int T) {
-  const TileShape sh = fp8_tile_shape(N, T);
-  const int kp = sh.W / sh.M, blocks = ((K / 128 + kp - 1) / kp) * T;
+int fp8_fused_passes(const RowShape& sh, int K, int T) {
+  if (T > kFusedMaxTokens) return 0;
+  const int blocks = ((K / 128 + sh.parts() - 1) / sh.parts()) * T;
   if (blocks > kTileQRows) return 0;
   const int per_wave = (blocks + sh.M - 1) / sh.M;
   return per_wave <= 4 ? 1 : per_wave <= 8 ? 2 : 4;
 }
 
-// Whether a block-128 call runs on fp8_tile_gemv_kernel: up to kFusedMaxTokens tokens (above that the split-K
-// GEMV, whose 64-row workgroups load each activation chunk once for 4 tiles, measured faster).
-bool fp8_tile_call(int N, int K, int T, int block) {
-  return block == 128 && T <= kFusedMaxTokens && fp8_tile_ok(N, K, T);
-}
-
-// Whether the block-128 GEMV can quantize its own activations: a tile call whose every wave's blocks fit its
-// LDS rows.
-bool fp8_fused_ok(int N, int K, int T, int block) {
-  return fp8_tile_call(N, K, T, block) && fp8_tile_passes(N, K, T) > 0;
-}
-
-// fp8_tile_gemv_kernel of shape (W, M): P fused quantization passes, or P = 0 when x comes quantized.
-template <int W, int M>
-void launch_tile_gemv(const Fp8Args& a, int P, dim3 grid, hipStream_t st) {
+// fp8_row_gemv_kernel of shape (W, M, TM): P fused quantization passes, or P = 0 when x comes quantized.
+template <int kBlock, int W, int M, int TM, bool kPair = false>
+void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st) {
+  const int sets = kPair ? a.N / 16 : a.N / 16 / TM;
   const dim3 threads(64 * W);
-  if (P == 1) hipLaunchKernelGGL((fp8_tile_gemv_kernel<true, W, M, 1>), grid, threads, 0, st, a);
-  else if (P == 2) hipLaunchKernelGGL((fp8_tile_gemv_kernel<true, W, M, 2>), grid, threads, 0, st, a);
-  else if (P == 4) {
-    if constexpr (16 * M <= kTileQRows) hipLaunchKernelGGL((fp8_tile_gemv_kernel<true, W, M, 4>), grid, threads, 0, st, a);
-  } else hipLaunchKernelGGL((fp8_tile_gemv_kernel<false, W, M, 1>), grid, threads, 0, st, a);
+  auto go = [&](auto kernel, int tokens = kTok) {
+    hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens), threads, 0, st, a);
+  };
+  if constexpr (M == 1 && !kPair)   // the shapes of more than 8 tokens
+    if (a.T > kTok) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
+  if (P == 0) go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair>);
+  if (P == 1) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair>);
+  if constexpr (8 * M <= kTileQRows)
+    if (P == 2) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 2, kPair>);
+  if constexpr (16 * M <= kTileQRows)
+    if (P == 4) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 4, kPair>);
 }
 
-// The product on quantized activations: the tile GEMV (block 128, T <= kFusedMaxTokens: no K split across
-// workgroups), the split-K GEMV (T <= 32) or the tiled GEMM, the latter two with K split over fp8_splits(N,
-// K, T) workgroups whose FP32 partial sums are added in split order: by the GEMV's last workgroup per tile
-// through the context's arrival counters and handoff buffer when they fit it (kTicketPartialBytes), else
-// written to `partial` (fp8_splits * T * N floats) and added by fp8_splitk_reduce_kernel.
-// x_fused: the BF16 input when the GEMV quantizes it itself (fp8_fused_ok), else null (q and sc given).
+template <int kBlock>
+void launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st) {
+  if (sh.W == 4 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 4, 1, 1>(a, P, st);
+  else if (sh.W == 8 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 8, 1, 1>(a, P, st);
+  else if (sh.W == 4 && sh.M == 1 && sh.TM == 2) launch_row_gemv<kBlock, 4, 1, 2>(a, P, st);
+  else if (sh.W == 8 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 8, 2, 1>(a, P, st);
+  else if (sh.W == 8 && sh.M == 2 && sh.TM == 2) launch_row_gemv<kBlock, 8, 2, 2>(a, P, st);
+  else if (sh.W == 16 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 16, 2, 1>(a, P, st);
+}
+
+// Whether the GEMV quantizes a plain call's activations itself (fp8_row_gemv_kernel, few tokens).
+bool fp8_fused_ok(int N, int K, int T) { return T <= kFusedMaxTokens && fp8_fused_passes(fp8_row_shape(N, K, T), K, T) > 0; }
+
+// fp8_quant_ordered_kernel: T tokens' codes and scales into buffers of T rounded up to 16 rows.
+int launch_quant_ordered(int block, const uint16_t* x, uint8_t* q, void* s, int T, int K, hipStream_t st) {
+  const int C = K / 128;
+  const dim3 grid((unsigned)(((int64_t)T * C + 15) / 16));
+  if (block == 32) hipLaunchKernelGGL(fp8_quant_ordered_kernel<32>, grid, dim3(256), 0, st, x, q, (uint8_t*)s, T, C);
+  else hipLaunchKernelGGL(fp8_quant_ordered_kernel<128>, grid, dim3(256), 0, st, x, q, (uint8_t*)s, T, C);
+  MX_LAUNCH_CHECK("fp8_quant_ordered_kernel");
+  return MX_OK;
+}
+
+// The product on quantized activations: the row GEMV (T <= 32: no K split across workgroups) or the tiled GEMM,
+// with K split over fp8_splits(N, K, T) workgroups whose FP32 partial sums go to `partial` (fp8_splits * T * N
+// floats) and are added in split order by fp8_splitk_reduce_kernel.
+// x_fused: the BF16 input when the GEMV quantizes it itself (fp8_fused_ok), else null (q and sc given); ordered: q
+// and sc as launch_quant_ordered wrote them.
 int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8_t* q, const void* sc, int T,
-                       uint16_t* y, float* trace, float* partial, mx_ctx* ctx, hipStream_t st,
-                       const uint16_t* x_fused = nullptr, int x_group_rows = 0) {
+                       uint16_t* y, float* trace, float* partial, hipStream_t st, const uint16_t* x_fused = nullptr,
+                       bool ordered = false, int x_group_rows = 0) {
   Fp8Args a{};
   a.blob = blob;
   a.N = N;
@@ -857,39 +826,13 @@ int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8
   a.trace = trace;
   a.partial = partial;
   a.x = x_fused;
-  if (x_fused) a.xq = reinterpret_cast<const uint8_t*>(x_fused);   // not read: B comes from LDS
-  if (fp8_tile_call(N, K, T, block)) {
-    const TileShape sh = fp8_tile_shape(N, T);
-    const dim3 grid(N / 16 / sh.M, (T + kTok - 1) / kTok);
-    const int P = x_fused ? fp8_tile_passes(N, K, T) : 0;
-    if (sh.W == 16) launch_tile_gemv<16, 2>(a, P, grid, st);
-    else if (sh.M == 2) launch_tile_gemv<8, 2>(a, P, grid, st);
-    else launch_tile_gemv<8, 1>(a, P, grid, st);
-    MX_LAUNCH_CHECK("fp8_tile_gemv_kernel");
-  } else if (T <= kGemvMaxTokens) {
-    const int splits = fp8_splits(N, K, T);
-    const dim3 grid(N / 64, (T + kTok - 1) / kTok, splits);
-    if (splits > 1 && (size_t)grid.x * grid.y <= MX_TICKETS &&
-        (uint64_t)splits * T * N * sizeof(float) <= kTicketPartialBytes) {
-      // this launch's half, and the other half's extent the previous launch wrote (restored by this launch)
-      const int h = ctx->handoff_half;
-      a.tickets = ctx->tickets;
-      a.handoff = ctx->handoff + (size_t)h * (MX_HANDOFF_BYTES / 4);
-      a.restore = reinterpret_cast<uint4*>(ctx->handoff + (size_t)(1 - h) * (MX_HANDOFF_BYTES / 4));
-      a.restore_n = (int64_t)(ctx->handoff_dirty[1 - h] / 16);
-      ctx->handoff_dirty[1 - h] = 0;
-      ctx->handoff_dirty[h] = ((uint64_t)splits * T * N * sizeof(float) + 15) / 16 * 16;
-      ctx->handoff_half = 1 - h;
-    }
-    if (block == 32) hipLaunchKernelGGL(fp8_gemv_kernel<32>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(fp8_gemv_kernel<128>, grid, dim3(256), 0, st, a);
-    MX_LAUNCH_CHECK("fp8_gemv_kernel");
-    if (splits > 1 && !a.tickets) {
-      const int64_t count = (int64_t)T * N;
-      hipLaunchKernelGGL(fp8_splitk_reduce_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, st,
-                         (const float*)partial, splits, count, y, trace);
-      MX_LAUNCH_CHECK("fp8_splitk_reduce_kernel");
-    }
+  a.ordered = ordered;
+  if (T <= kGemvMaxTokens) {
+    const RowShape sh = fp8_row_shape(N, K, T);
+    const int P = x_fused ? fp8_fused_passes(sh, K, T) : 0;
+    if (block == 32) launch_row_gemv<32>(sh, a, P, st);
+    else launch_row_gemv<128>(sh, a, P, st);
+    MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
   } else {
     const int splits = fp8_splits(N, K, T);
     const dim3 grid((N / 64 + 3) / 4, (T + kGemmTok - 1) / kGemmTok, splits);
@@ -903,19 +846,6 @@ int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8
     }
   }
   return MX_OK;
-}
-
-// SwiGLU of the FP8 expert, one element per thread (the gate/up kernel of the MXFP4 path applies the
-// same mxd::swiglu_element in its epilogue).
-__global__ void swiglu_kernel(const uint16_t* __restrict__ w1, const uint16_t* __restrict__ w3, int T, int I,
-                              float limit, const float* __restrict__ route_w, uint16_t* __restrict__ din,
-                              float* __restrict__ trace) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)T * I) return;
-  const int t = (int)(i / I);
-  const float v = mxd::swiglu_element(w1[i], w3[i], limit, route_w != nullptr, route_w ? route_w[t] : 1.f,
-                                      trace ? trace + i * 5 : nullptr);
-  din[i] = (uint16_t)mx::bf16_bits(v);
 }
 
 }  // namespace
@@ -974,24 +904,28 @@ int mx_fp8_projection(mx_ctx* ctx, const void* tiled, int32_t N, int32_t K, int3
                  ((uintptr_t)trace & 15) == 0,
              "mx_fp8_projection: tiled 256-byte, x 16-byte, y 8-byte and trace 16-byte alignment required");
   hipStream_t st = as_stream(stream);
-  const uint64_t q_b = ((uint64_t)T * K + 255) & ~255ull;
-  const uint64_t s_b = ((block == 32 ? (uint64_t)T * (K / 32) : (uint64_t)T * (K / 128) * 4) + 255) & ~255ull;
-  const uint64_t p_b = fp8_tile_call(N, K, T, block) ? 0 : (uint64_t)fp8_splits(N, K, T) * T * N * 4;
+  // the decode GEMV's own codes come in its load order, in whole tiles of 16 tokens
+  const bool ordered = !q_out && !s_out && T <= kGemvMaxTokens;
+  const uint64_t rows = ordered ? (T + kTok - 1) / kTok * kTok : T;
+  const uint64_t q_b = (rows * K + 255) & ~255ull, s_b = (rows * (K / 32) + 255) & ~255ull;   // 4 scale bytes a chunk
+  const int splits = fp8_splits(N, K, T);
+  const uint64_t p_b = splits > 1 ? (uint64_t)splits * T * N * 4 : 0;
   void* base = nullptr;
   if (int s = scratch(ctx, q_b + s_b + p_b + 256, &base)) return s;
   uint8_t* q = q_out ? q_out : (uint8_t*)base;
   void* sc = s_out ? s_out : (void*)((uint8_t*)base + q_b);
   MX_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)sc & 3) == 0, "mx_fp8_projection: q 16-byte, s 4-byte aligned");
   float* partial = (float*)((uint8_t*)base + q_b + s_b);
-  if (!q_out && !s_out && fp8_fused_ok(N, K, T, block))   // the GEMV quantizes x itself
-    return launch_fp8_product((const uint8_t*)tiled, N, K, block, nullptr, nullptr, T, y, trace, partial, ctx, st,
-                              x);
-  if (block == 32) {
+  if (!q_out && !s_out && fp8_fused_ok(N, K, T))   // the GEMV quantizes x itself
+    return launch_fp8_product((const uint8_t*)tiled, N, K, block, nullptr, nullptr, T, y, trace, partial, st, x);
+  if (ordered) {
+    if (int s = launch_quant_ordered(block, x, q, sc, T, K, st)) return s;
+  } else if (block == 32) {
     if (int s = mx_act_quant32(ctx, x, q, (uint8_t*)sc, T, K, stream)) return s;
   } else {
     if (int s = mx_act_quant128(ctx, x, q, (float*)sc, T, K, stream)) return s;
   }
-  return launch_fp8_product((const uint8_t*)tiled, N, K, block, q, sc, T, y, trace, partial, ctx, st);
+  return launch_fp8_product((const uint8_t*)tiled, N, K, block, q, sc, T, y, trace, partial, st, nullptr, ordered);
 }
 
 int mx_fp8_grouped_projection(mx_ctx* ctx, const void* tiled, int32_t groups, int32_t rows, int32_t K,
@@ -1008,10 +942,8 @@ int mx_fp8_grouped_projection(mx_ctx* ctx, const void* tiled, int32_t groups, in
   MX_REQUIRE(((uintptr_t)tiled & 255) == 0 && ((uintptr_t)q & 15) == 0 && ((uintptr_t)s & 3) == 0 &&
                  ((uintptr_t)y & 7) == 0 && ((uintptr_t)trace & 15) == 0,
              "mx_fp8_grouped_projection: tiled 256-byte, q 16-byte, s 4-byte, y 8-byte, trace 16-byte alignment");
-  void* base = nullptr;
-  if (int st = scratch(ctx, (uint64_t)fp8_splits(N, K, T) * T * N * 4 + 256, &base)) return st;
-  return launch_fp8_product((const uint8_t*)tiled, N, K, 32, q, s, T, y, trace, (float*)base, ctx,
-                            as_stream(stream), nullptr, rows);
+  return launch_fp8_product((const uint8_t*)tiled, N, K, 32, q, s, T, y, trace, nullptr, as_stream(stream), nullptr,
+                            false, rows);
 }
 
 int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const void* w2, int32_t H, int32_t I,
@@ -1029,42 +961,58 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
              "x and y must be 16-byte aligned device pointers");
   hipStream_t st = as_stream(stream);
   auto r256 = [](uint64_t b) { return (b + 255) & ~255ull; };
-  const uint64_t sizes[7] = {r256((uint64_t)T * H),     r256((uint64_t)T * H / 32), r256((uint64_t)T * I * 2),
-                             r256((uint64_t)T * I * 2), r256((uint64_t)T * I * 2),  r256((uint64_t)T * I),
-                             r256((uint64_t)T * I / 32)};
-  const uint64_t p_b = (uint64_t)std::max(fp8_splits(I, H, T) * I, fp8_splits(H, I, T) * H) * T * 4;
-  uint64_t total = p_b;
+  const uint64_t sizes[5] = {r256((uint64_t)kTok * H), r256((uint64_t)kTok * H / 32), r256((uint64_t)T * I * 2),
+                             r256((uint64_t)kTok * I), r256((uint64_t)kTok * I / 32)};
+  uint64_t total = 0;
   for (uint64_t b : sizes) total += b;
   void* base = nullptr;
   if (int s = scratch(ctx, total, &base)) return s;
   uint8_t* cur = (uint8_t*)base;
-  uint8_t* buf[7];
-  for (int i = 0; i < 7; ++i) {
+  uint8_t* buf[5];
+  for (int i = 0; i < 5; ++i) {
     buf[i] = cur;
     cur += sizes[i];
   }
-  float* partial = (float*)cur;
   uint8_t* q = (stages && stages->q) ? stages->q : buf[0];
   uint8_t* s = (stages && stages->s) ? stages->s : buf[1];
-  uint16_t* b1 = (stages && stages->w1) ? stages->w1 : (uint16_t*)buf[2];
-  uint16_t* b3 = (stages && stages->w3) ? stages->w3 : (uint16_t*)buf[3];
-  uint16_t* din = (stages && stages->down_input) ? stages->down_input : (uint16_t*)buf[4];
-  uint8_t* dq = (stages && stages->down_q) ? stages->down_q : buf[5];
-  uint8_t* ds = (stages && stages->down_s) ? stages->down_s : buf[6];
-  float* trace = stages ? stages->trace : nullptr;
-  MX_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)dq & 15) == 0 && ((uintptr_t)b1 & 7) == 0 &&
-                 ((uintptr_t)b3 & 7) == 0 && ((uintptr_t)din & 3) == 0 && ((uintptr_t)s & 3) == 0 &&
+  uint16_t* din = (stages && stages->down_input) ? stages->down_input : (uint16_t*)buf[2];
+  uint8_t* dq = (stages && stages->down_q) ? stages->down_q : buf[3];
+  uint8_t* ds = (stages && stages->down_s) ? stages->down_s : buf[4];
+  Fp8Args a{};
+  a.blob = (const uint8_t*)w1;
+  a.blob2 = (const uint8_t*)w3;
+  a.N = I;
+  a.K = H;
+  a.T = T;
+  a.xq = q;
+  a.xs = s;
+  a.x_stride = H;
+  a.y = stages ? stages->w1 : nullptr;
+  a.y3 = stages ? stages->w3 : nullptr;
+  a.din = din;
+  a.swiglu_trace = stages ? stages->trace : nullptr;
+  a.route_w = route_w;
+  a.limit = limit;
+  MX_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)dq & 15) == 0 && ((uintptr_t)a.y & 7) == 0 &&
+                 ((uintptr_t)a.y3 & 7) == 0 && ((uintptr_t)din & 3) == 0 && ((uintptr_t)s & 3) == 0 &&
                  ((uintptr_t)ds & 3) == 0,
              "stage buffers: q/down_q 16-byte, w1/w3 8-byte, scales and down_input 4-byte aligned");
-  if (int e = mx_act_quant32(ctx, x, q, s, T, H, stream)) return e;
-  if (int e = launch_fp8_product((const uint8_t*)w1, I, H, 32, q, s, T, b1, nullptr, partial, ctx, st)) return e;
-  if (int e = launch_fp8_product((const uint8_t*)w3, I, H, 32, q, s, T, b3, nullptr, partial, ctx, st)) return e;
-  const int64_t n = (int64_t)T * I;
-  hipLaunchKernelGGL(swiglu_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const uint16_t*)b1,
-                     (const uint16_t*)b3, T, I, limit, route_w, din, trace);
-  MX_LAUNCH_CHECK("swiglu_kernel");
-  if (int e = mx_act_quant32(ctx, din, dq, ds, T, I, stream)) return e;
-  return launch_fp8_product((const uint8_t*)w2, H, I, 32, dq, ds, T, y, nullptr, partial, ctx, st);
+  // few tokens: each launch quantizes its own input, unless the caller asks for those codes (or, for the down
+  // input, gives a buffer that 16-byte loads cannot read); more tokens: codes in the GEMV's load order
+  const bool own_q = !stages || (!stages->q && !stages->s);
+  const int p1 = own_q ? fp8_fused_passes(kPairShape, H, T) : 0;
+  a.ordered = own_q;
+  if (p1) a.x = x;
+  else if (int e = own_q ? launch_quant_ordered(32, x, q, s, T, H, st) : mx_act_quant32(ctx, x, q, s, T, H, stream))
+    return e;
+  launch_row_gemv<32, kPairShape.W, 1, 2, true>(a, p1, st);
+  MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
+  const bool own_dq = (!stages || (!stages->down_q && !stages->down_s)) && ((uintptr_t)din & 15) == 0;
+  if (own_dq && fp8_fused_ok(H, I, T))
+    return launch_fp8_product((const uint8_t*)w2, H, I, 32, nullptr, nullptr, T, y, nullptr, nullptr, st, din);
+  if (int e = own_dq ? launch_quant_ordered(32, din, dq, ds, T, I, st) : mx_act_quant32(ctx, din, dq, ds, T, I, stream))
+    return e;
+  return launch_fp8_product((const uint8_t*)w2, H, I, 32, dq, ds, T, y, nullptr, nullptr, st, nullptr, own_dq);
 }
 
 }  // extern "C"
