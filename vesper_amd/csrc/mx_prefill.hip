@@ -40,7 +40,7 @@ constexpr int kMaxTopK = 32;
 struct PrefillPlan {
   int32_t* counts;      // [E + 1] pairs per slot (slot E = shared expert)
   int32_t* row0;        // [E + 1] first row of each slot
-  int32_t* tile_info;   // [max_tiles][4]: slot, first row, rows, unused
+  int32_t* tile_info;   // [max_tiles][4]: slot, first row, rows, 1 if it is the slot's only tile
   int32_t* n_tiles;     // [1]
   int32_t* sorted_tok;  // [rows] token of each row
   float* sorted_w;      // [rows] route weight of each row
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(64) void offsets_kernel(PrefillPlan p, int E, int T
         info[0] = s;
         info[1] = r0 + j * kTileRows;
         info[2] = min(kTileRows, cnt - j * kTileRows);
-        info[3] = 0;
+        info[3] = tiles == 1;
       }
     }
     row_carry += __shfl(rs, 63, 64);
@@ -191,6 +191,7 @@ struct GemmArgs {
   const uint8_t* const* tiles;   // [E + 1] tiled expert blobs
   PrefillPlan plan;
   int H, I, E;
+  int shared_tiles;              // tiles of the shared expert, the list's last (0: none)
   float limit;
   const float* silu;             // [mxd::kSiluEntries] the layer's SiLU table
   const uint8_t* xq;             // [T][H] E4M3 codes of the tokens
@@ -200,6 +201,17 @@ struct GemmArgs {
   uint8_t* ds;                   // [rows][I / 32]
   uint16_t* out;                 // [T][k + 1][H] expert outputs (BF16), token-major (plan.row_dest)
 };
+
+// The tile that launch row y takes of a list whose last `shared` entries are the shared expert's. Those are full tiles,
+// whose workgroups run several times longer than most (few rows per expert): where they are too few to fill the CUs
+// they go first -- last, they would hold the launch open alone -- and where they fill them they stay last.
+// Gate/up + down, us: 1000 tokens of the 384-expert model 1912 -> 1835, 300 and 2000 of the 256-expert one 1374-1423 ->
+// 1269 and 2612-2647 -> 2549; 4096 tokens (32 tiles, 256 and 448 workgroups) 3585-3596 last, 3627 first, and 3638-3653
+// spread over the launch.
+__device__ __forceinline__ int tile_of_row(int y, int total, int shared) {
+  if (shared * (int)gridDim.x >= 256) return y;
+  return y < shared ? total - shared + y : y - shared;
+}
 
 using mxd::copy_barrier;
 using mxd::global_to_lds16;
@@ -256,8 +268,9 @@ static_assert(kLdsBytes <= 160 * 1024 && 2 * kTileRows * kEpiRowG * 2 <= kLdsByt
 // segments of the down output to the token-major output rows (plan.row_dest).
 __global__ __launch_bounds__(kGThreads) void grouped_down_kernel(GemmArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
-  const int ti = blockIdx.y;
-  if (ti >= *a.plan.n_tiles) return;
+  const int total = *a.plan.n_tiles;
+  if ((int)blockIdx.y >= total) return;
+  const int ti = __builtin_amdgcn_readfirstlane(tile_of_row(blockIdx.y, total, a.shared_tiles));
   const int32_t* info = a.plan.tile_info + (size_t)ti * 4;
   const int slot = info[0], row0 = info[1], rows = info[2];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -284,6 +297,7 @@ __global__ __launch_bounds__(kGThreads) void grouped_down_kernel(GemmArgs a) {
     // (both blocks of each) and the scale words of rows 32p .. 32p + 31. Rows past the tile repeat its last
     // row; groups past the last repeat it. The activation offsets fit 32 bits (the host bounds the buffers).
     const int pw = wave - 8;
+    const bool once = __builtin_amdgcn_readfirstlane(info[3]) != 0;
     const uint8_t* wsrc[2];
     const uint8_t* ssrc[2];
 #pragma unroll
@@ -305,9 +319,12 @@ __global__ __launch_bounds__(kGThreads) void grouped_down_kernel(GemmArgs a) {
     auto copy = [&](int c) {
       const uint32_t st = lds0 + (uint32_t)(c % kStages) * kStageBytes;
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        global_to_lds16(wsrc[i >> 2] + (size_t)c * 4096 + (i & 3) * 1024,
-                        __builtin_amdgcn_readfirstlane(st + kStageA + (8 * pw + i) * 1024));
+      for (int i = 0; i < 8; ++i) {
+        const uint8_t* w = wsrc[i >> 2] + (size_t)c * 4096 + (i & 3) * 1024;
+        const uint32_t wl = __builtin_amdgcn_readfirstlane(st + kStageA + (8 * pw + i) * 1024);
+        if (once) mxd::global_to_lds16_nt(w, wl);   // read by this tile alone (2 % of the launch; none in gate/up)
+        else global_to_lds16(w, wl);
+      }
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         global_to_lds4(ssrc[i] + (size_t)c * 256, __builtin_amdgcn_readfirstlane(st + kStageAS + 256 * (2 * pw + i)));
@@ -418,24 +435,31 @@ __global__ __launch_bounds__(kGThreads) void grouped_down_kernel(GemmArgs a) {
 //
 // grid (ceil(I / 256), tiles), 512 threads: 8 waves, wave w one group of 32 intermediate rows (4 MFMA
 // tiles, W1 rows 8t + 0..7 and the same W3 rows in tile t) for all 128 rows of the tile, 128 accumulator
-// registers. Every wave copies its share of chunk c + 1's operands global -> LDS (global_load_lds, nine
-// instructions: its group's four weight pieces and scale words, and token tile w's four BF16 activation
-// blocks) into a 2-stage ring; a step waits for this wave's copies of chunk c, meets the barrier and
-// multiplies chunk c, issuing chunk c + 1's copies a block at a time between its blocks. (Half-chunk steps
-// through a 4-stage ring, which copy three steps ahead, and FP8 activations through a 3-stage ring,
-// converted per wave, both measured slower: per-step costs -- the barrier, the first LDS reads, the last
-// additions -- and the conversions outweigh the deeper prefetch.) Operands come from LDS with the bf16
+// registers. Every wave copies its share of a chunk's operands global -> LDS (global_load_lds: its group's four
+// weight pieces and scale words, and token tile w's four BF16 activation blocks if the tile is live) into a ring of S
+// stages (xstages: 2 for full tiles, up to 4 where few token tiles are live); a step waits for this wave's copies of
+// chunk c, meets the barrier and multiplies chunk c, issuing chunk c + S - 1's copies a block at a time between its
+// blocks. (For full tiles, half-chunk steps through a 4-stage ring and FP8 activations through a 3-stage ring,
+// converted per wave, both measured slower: per-step costs -- the barrier, the first LDS reads, the last additions --
+// and the conversions outweigh the deeper prefetch.) Operands come from LDS with the bf16
 // MFMA's lane map (A lane (m, q) = row m, K 8q..8q+7 of a block: word q of lane (m, b)'s 16 bytes in the
 // tiled layout; B lane (n, q) = token n, the same K: the copy puts them at lane slot 16 q + n of the (token
 // tile, block) KB). The reads are plain LDS loads: the copies are inline assembly, which the compiler does
 // not see writing LDS, so it places no wait for them before a read -- the wave's own vmcnt wait and the
 // barrier at the top of each step order them.
 constexpr int kXThreads = 512;
-constexpr int kXStages = 2;
 // a stage: the 8 groups' weight tiles (group w, tile t at 1 KB x (4 w + t)), their scale words (256 B per
-// group), then the activations: token tile u, block b at 1 KB x (4 u + b)
-constexpr int kXStageA = 0, kXStageAS = 32768, kXStageB = 34816, kXStageBytes = 67584;
-static_assert(kXStages * kXStageBytes <= 160 * 1024 && 2 * kTileRows * kEpiRowG * 2 <= kXStages * kXStageBytes,
+// group), then the activations of the tile's live token tiles: token tile u, block b at 1 KB x (4 u + b)
+constexpr int kXStageA = 0, kXStageAS = 32768, kXStageB = 34816;
+constexpr int xstage_bytes(int live) { return kXStageB + 4096 * live; }
+// stages in the ring with `live` token tiles: as many as the LDS holds, at most 4
+constexpr int xstages(int live) { return 160 * 1024 / xstage_bytes(live) < 4 ? 160 * 1024 / xstage_bytes(live) : 4; }
+constexpr int xlds_bytes(int live) { return xstages(live) * xstage_bytes(live); }
+constexpr int xlds_max(int live = 8) {
+  return live == 0 ? 0 : xlds_bytes(live) > xlds_max(live - 1) ? xlds_bytes(live) : xlds_max(live - 1);
+}
+constexpr int kXLdsBytes = xlds_max();
+static_assert(xstages(8) >= 2 && kXLdsBytes <= 160 * 1024 && 2 * kTileRows * kEpiRowG * 2 <= kXLdsBytes,
               "exact gate/up LDS layout");
 
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
@@ -499,46 +523,59 @@ struct ExactStream {
   uint32_t lds0, la, las, lb;
   int wave, C;
   bool active;
-  // block b's share of the copies of chunk c: weight piece b and activation block b (and the scale words
-  // with block 0)
-  __device__ __forceinline__ void copy_block(int c, int b) const {
-    const uint32_t st = lds0 + (uint32_t)(c % kXStages) * kXStageBytes;
-    global_to_lds16(wsrc + (size_t)c * 4096 + b * 1024,
-                    __builtin_amdgcn_readfirstlane(st + kXStageA + (4 * wave + b) * 1024));
+  // block b's share of the copies of chunk c into the stage at LDS address st: weight piece b and, by the waves of
+  // live token tiles, activation block b (and the scale words with block 0)
+  __device__ __forceinline__ void copy_block(int c, int b, uint32_t st, bool acts) const {
+    const uint32_t wl = __builtin_amdgcn_readfirstlane(st + kXStageA + (4 * wave + b) * 1024);
+    global_to_lds16(wsrc + (size_t)c * 4096 + b * 1024, wl);
     if (b == 0) global_to_lds4(ssrc + (size_t)c * 256, __builtin_amdgcn_readfirstlane(st + kXStageAS + 256 * wave));
-    global_to_lds16(xbase + (size_t)c * 256 + boff + 64 * b,
-                    __builtin_amdgcn_readfirstlane(st + kXStageB + (4 * wave + b) * 1024));
+    if (acts)
+      global_to_lds16(xbase + (size_t)c * 256 + boff + 64 * b,
+                      __builtin_amdgcn_readfirstlane(st + kXStageB + (4 * wave + b) * 1024));
   }
   // all of chunk c's copies
-  __device__ __forceinline__ void copy(int c) const {
+  __device__ __forceinline__ void copy(int c, uint32_t st, bool acts) const {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) copy_block(c, b);
+    for (int b = 0; b < 4; ++b) copy_block(c, b, st, acts);
   }
 };
 
 // The K loop for a tile with L live 16-row token tiles (L is a template argument so that the token-tile loop
-// has no per-tile branches).
+// has no per-tile branches). The ring has xstages(L) stages, S - 1 chunks copied ahead: the fewer the live tiles, the
+// shorter a chunk's work and the more the copies' latency shows, and the smaller its stage. (With two
+// stages for every L and every token tile's rows copied, gate/up of 1000 tokens over 384 experts, 16 rows each, took
+// 1198 us, now 1064; 4096 tokens of Zipf routing, whose time goes to full tiles, 2673 and 2682.)
 template <int L>
 __device__ __forceinline__ void exact_stream(const ExactStream& s, v4f (&acc)[4][8]) {
+  constexpr int S = xstages(L), kBytes = xstage_bytes(L);
   const uint32_t k23 = 23;
-  s.copy(0);
+  const bool acts = s.wave < L;   // this wave copies a live token tile's rows
+#pragma unroll
+  for (int c = 0; c < S - 1; ++c)
+    if (c < s.C) s.copy(c, s.lds0 + c * kBytes, acts);
+  uint32_t slot = 0, next = S - 1;   // the ring slots of chunk c and of chunk c + S - 1
   for (int c = 0; c < s.C; ++c) {
-    __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));   // this wave's copies of chunk c have landed
+    // this wave's copies of chunk c have landed (those of chunks c + 1 .. c + S - 2 may be in flight)
+    if (S == 2 || c + S - 2 >= s.C) __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));
+    else if (acts) __builtin_amdgcn_s_waitcnt(vm_wait_imm((S - 2) * 9));
+    else __builtin_amdgcn_s_waitcnt(vm_wait_imm((S - 2) * 5));
     copy_barrier();   // every wave's copies of chunk c are visible; chunk c - 1's stage is free
     // the next chunk's copies go out a block at a time between this chunk's blocks: issued together right
     // after the barrier, all eight waves' 72 copies queue at the CU's memory unit at once and each wave
     // stalled 750-1,060 clocks a chunk before its first conversion (per-wave clock stamps of a probe build)
-    const bool more = c + 1 < s.C;
+    const bool more = c + S - 1 < s.C;
+    const uint32_t so = slot * kBytes, st = s.lds0 + next * kBytes;
+    slot = slot == S - 1 ? 0 : slot + 1;
+    next = next == S - 1 ? 0 : next + 1;
     if (!s.active) {
-      if (more) s.copy(c + 1);
+      if (more) s.copy(c + S - 1, st, acts);
       continue;
     }
-    const uint32_t so = (uint32_t)(c % kXStages) * kXStageBytes;
     uint32_t w[4][4], sw[4];
     lds_read_weights(s.la + so, s.las + so, w, sw);
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      if (more) s.copy_block(c + 1, b);
+      if (more) s.copy_block(c + S - 1, b, st, acts);
       const float ws[4] = {e8m0_scale<0>(sw[b], k23), e8m0_scale<1>(sw[b], k23), e8m0_scale<2>(sw[b], k23),
                            e8m0_scale<3>(sw[b], k23)};
       v8bf av[4];
@@ -573,9 +610,10 @@ __device__ __forceinline__ void exact_stream(const ExactStream& s, v4f (&acc)[4]
 }
 
 __global__ __launch_bounds__(kXThreads) void gateup_exact_kernel(GemmArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kXStages * kXStageBytes];
-  const int ti = blockIdx.y;
-  if (ti >= *a.plan.n_tiles) return;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kXLdsBytes];
+  const int total = *a.plan.n_tiles;
+  if ((int)blockIdx.y >= total) return;
+  const int ti = __builtin_amdgcn_readfirstlane(tile_of_row(blockIdx.y, total, a.shared_tiles));
   const int32_t* info = a.plan.tile_info + (size_t)ti * 4;
   const int slot = info[0], row0 = info[1], rows = info[2];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -890,6 +928,7 @@ int mx_moe_prefill(mx_layer* layer, const uint16_t* x, int32_t T, const int32_t*
   a.H = H;
   a.I = I;
   a.E = E;
+  a.shared_tiles = v.has_shared ? (T + kTileRows - 1) / kTileRows : 0;
   a.limit = c.swiglu_limit;
   a.silu = v.silu;
   a.xq = b + ws.xq;
