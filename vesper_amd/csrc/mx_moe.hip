@@ -1183,6 +1183,123 @@ __global__ __launch_bounds__(256) void router_kernel(RouterArgs a) {
   }
 }
 
+// Router GEMV of many tokens: grid (ceil(E / 8) ceil(T / 8)), 256 threads; a workgroup computes 8 experts for 8 tokens,
+// so that a load of W_r serves 8 tokens and a load of x 8 experts. (router_kernel reads a token's row once per expert:
+// 3.9 GB from L2 at 1000 tokens of 384 experts, 251 us; here 1.5 GB, 78 us, 36 of them arithmetic.) Every (expert, token) sum is
+// router_kernel's, bit for bit: the thread's FMAs run in the same order, the wave's 64 sums are added in the same
+// balanced tree (lane pairs 1, 2, 4, 8, 16, 32 apart; addition commutes), halving the values a lane carries at each
+// step so that 64 trees take 63 additions a lane instead of 384, and the four waves' parts in wave order.
+constexpr int kRouterTile = 8;
+
+template <int kXor>
+__device__ __forceinline__ float lane_xor(float v) {
+  const int b = __float_as_int(v);
+  if constexpr (kXor == 1) return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0xB1, 0xF, 0xF, false));   // [1,0,3,2]
+  if constexpr (kXor == 2) return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x4E, 0xF, 0xF, false));   // [2,3,0,1]
+  if constexpr (kXor == 4 || kXor == 8 || kXor == 16) return __int_as_float(swizzle_xor<kXor>(b));
+  return __shfl_xor(v, kXor, 64);
+}
+
+// One tree level: of 2 kHalf values a lane keeps kHalf, the upper ones where its bit kXor is set, each added to its
+// partner lane's.
+template <int kXor, int kHalf>
+__device__ __forceinline__ void tree_level(float (&v)[kRouterTile * kRouterTile], int lane) {
+  const bool upper = lane & kXor;
+#pragma unroll
+  for (int j = 0; j < kHalf; ++j) {
+    const float keep = upper ? v[j + kHalf] : v[j], send = upper ? v[j] : v[j + kHalf];
+    v[j] = keep + lane_xor<kXor>(send);
+  }
+}
+
+__global__ __launch_bounds__(256) void router_tile_kernel(RouterArgs a) {
+  constexpr int kN = kRouterTile;
+  const int egroups = (a.E + kN - 1) / kN;   // expert groups fastest: an XCD keeps meeting the same rows of W_r
+  const int e0 = (int)(blockIdx.x % egroups) * kN, t0 = (int)(blockIdx.x / egroups) * kN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // experts and tokens past the last repeat it; their sums are dropped
+  const float* w[kN];
+  const uint16_t* x[kN];
+#pragma unroll
+  for (int i = 0; i < kN; ++i) {
+    w[i] = a.W + (size_t)min(e0 + i, a.E - 1) * a.H;
+    x[i] = a.x + (size_t)min(t0 + i, a.T - 1) * a.H;
+  }
+  float acc[kN * kN];   // [expert][token]
+#pragma unroll
+  for (int i = 0; i < kN * kN; ++i) acc[i] = 0.f;
+  // the next 1024 columns' operands are loaded under this step's FMAs (110 -> 78 us); past the end the last ones again
+  float4 wn[kN];
+  uint2 xn[kN];
+  {
+    const int k = min(tid * 4, a.H - 4);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) wn[i] = *reinterpret_cast<const float4*>(w[i] + k);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) xn[i] = *reinterpret_cast<const uint2*>(x[i] + k);
+  }
+  for (int k = tid * 4; k < a.H; k += 1024) {
+    float4 wv[kN];
+    uint2 xb[kN];
+    const int kn = min(k + 1024, a.H - 4);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      wv[i] = wn[i];
+      xb[i] = xn[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kN; ++i) wn[i] = *reinterpret_cast<const float4*>(w[i] + kn);
+#pragma unroll
+    for (int i = 0; i < kN; ++i) xn[i] = *reinterpret_cast<const uint2*>(x[i] + kn);
+#pragma unroll
+    for (int t = 0; t < kN; ++t) {
+      const float x0 = mx::bf16_value(xb[t].x & 0xFFFFu), x1 = mx::bf16_value(xb[t].x >> 16);
+      const float x2 = mx::bf16_value(xb[t].y & 0xFFFFu), x3 = mx::bf16_value(xb[t].y >> 16);
+#pragma unroll
+      for (int e = 0; e < kN; ++e) {
+        float v = acc[e * kN + t];
+        v = fmaf(wv[e].x, x0, v);
+        v = fmaf(wv[e].y, x1, v);
+        v = fmaf(wv[e].z, x2, v);
+        acc[e * kN + t] = fmaf(wv[e].w, x3, v);
+      }
+    }
+  }
+  tree_level<1, 32>(acc, lane);
+  tree_level<2, 16>(acc, lane);
+  tree_level<4, 8>(acc, lane);
+  tree_level<8, 4>(acc, lane);
+  tree_level<16, 2>(acc, lane);
+  tree_level<32, 1>(acc, lane);
+  // the lane's value: its lane number's bits, reversed
+  __shared__ float part[4][kN * kN];
+  part[wave][__brev((uint32_t)lane) >> 26] = acc[0];
+  __syncthreads();
+  const int e = e0 + tid / kN, t = t0 + tid % kN;
+  if (tid < kN * kN && e < a.E && t < a.T) {
+    const float z = ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
+    const size_t o = (size_t)t * a.E + e;
+    a.logits[o] = z;
+    const float s = score_of(z, a.score_func);
+    if (a.scores) a.scores[o] = s;
+    if (a.selection) a.selection[o] = a.bias ? s + a.bias[e] : s;
+  }
+}
+
+// The router's logits (and scores and selection values) of T tokens, by either kernel with the same bits. us at 17 / 24
+// / 32 / 64 / 333 tokens: 256 experts x 7168 9.8 / 10.0 / 11.9 / 19.8 / 81 with an expert a workgroup, 10.4 / 10.3 / 10.5 /
+// 10.9 / 29.5 with 8 x 8 tiles; 384 x 5120 10.1 / 10.8 / 12.7 / 22.1 / 91 and 8.6 / 8.6 / 8.8 / 10.3 / 28.9.
+int launch_router(const RouterArgs& r, hipStream_t st) {
+  if (r.T > 24)
+    hipLaunchKernelGGL(router_tile_kernel,
+                       dim3((unsigned)((r.E + kRouterTile - 1) / kRouterTile) * (unsigned)((r.T + kRouterTile - 1) / kRouterTile)),
+                       dim3(256), 0, st, r);
+  else
+    hipLaunchKernelGGL(router_kernel, dim3(r.E, (r.T + kMaxTokens - 1) / kMaxTokens), dim3(256), 0, st, r);
+  MX_LAUNCH_CHECK("router_kernel");
+  return MX_OK;
+}
+
 // Sum the 4 waves' partial tiles in wave order; wave w returns tile w's accumulator.
 __device__ __forceinline__ v4f reduce_tiles(const v4f (&acc)[kTiles], int wave, int lane, float (*red)[kTiles][64][4]) {
 #pragma unroll
@@ -2268,8 +2385,7 @@ int mx_router(mx_ctx* ctx, const float* W, const float* bias, const uint16_t* x,
   r.logits = out->logits;
   r.scores = scores;
   r.selection = selection;
-  hipLaunchKernelGGL(router_kernel, dim3(E, (T + kMaxTokens - 1) / kMaxTokens), dim3(256), 0, st, r);
-  MX_LAUNCH_CHECK("router_kernel");
+  if (int s = launch_router(r, st)) return s;
   TopkOut o{out->indices, out->weights, out->raw, out->denominator, out->tied};
   hipLaunchKernelGGL(topk_kernel, dim3((T + 3) / 4), dim3(256), 0, st, (const float*)selection, (const float*)scores,
                      T, E, k, route_scale, o);
@@ -2292,9 +2408,7 @@ int mx_gate_project(mx_ctx* ctx, const float* W, const uint16_t* x, int32_t T, i
   r.H = H;
   r.E = E;
   r.logits = logits;
-  hipLaunchKernelGGL(router_kernel, dim3(E, (T + kMaxTokens - 1) / kMaxTokens), dim3(256), 0, as_stream(stream), r);
-  MX_LAUNCH_CHECK("router_kernel");
-  return MX_OK;
+  return launch_router(r, as_stream(stream));
 }
 
 int mx_router_postprocess(mx_ctx* ctx, const float* logits, const float* bias, int32_t T, int32_t E, int32_t k,
