@@ -22,7 +22,7 @@
 //     its 8 intermediate positions: h = silu(g) * u (* route weight) in FP32 (optionally written out with g
 //     and u), and h as two BF16 terms hi + lo for the down product (hi = bf16(h), lo = bf16(h - hi): their
 //     sum holds h to about 16 significant bits);
-//   down (H/64 row blocks, 256 threads): W2 rows against hi and lo (two MFMAs per step), the four waves'
+//   down (H/32 row pairs of tiles, 8 waves): W2 rows against hi and lo (two MFMAs per step), the eight waves'
 //     sums added in wave order and rounded once to BF16.
 // Every sum runs in a fixed order (MFMA chains per wave, then waves), independent of T and of scheduling, so
 // a token's result does not depend on the batch it runs in.
@@ -81,58 +81,6 @@ __device__ __forceinline__ v8bf fp4_word_bf16(uint32_t word, uint32_t code) {
 
 __device__ __forceinline__ uint32_t word_of(const uint4 v, int r) {
   return r == 0 ? v.x : r == 1 ? v.y : r == 2 ? v.z : v.w;
-}
-
-// One 128-wide K chunk of a 4-tile weight group against up to 16 tokens: 4 MFMAs per tile, one per word.
-// w[t] = tile t's 16 bytes of this lane, sw = its scale word (byte t = tile t), xv[r] = the tokens' BF16
-// operand for word r; acc[t] accumulates tile t.
-template <int kTerms>
-__device__ __forceinline__ void chunk_mfma(const uint4 (&w)[4], uint32_t sw, const uint4 (&xv)[kTerms][4],
-                                           v4f (&acc)[4]) {
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const uint32_t code = (sw >> (8 * t)) & 0xFF;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const v8bf a = fp4_word_bf16(word_of(w[t], r), code);
-#pragma unroll
-      for (int term = 0; term < kTerms; ++term)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(v8bf, xv[term][r]), acc[t], 0, 0, 0);
-    }
-  }
-}
-
-// The wave's chunks [c0, c1) of a 4-tile group whose chunk c starts at wp + c * 4096 (tile t at + t * 1024,
-// lane at + 16 lane) with scale words at sp + c * 256 (+ 4 lane); act(term, c, r) = the address of this
-// lane's 16-byte activation operand. Loads run kRing chunks ahead in a statically indexed ring.
-template <int kTerms, typename Act>
-__device__ __forceinline__ void stream_group(const uint8_t* wp, const uint8_t* sp, int c0, int c1, Act act,
-                                             v4f (&acc)[4]) {
-  uint4 w[kRing][4];
-  uint32_t sw[kRing];
-  uint4 xv[kRing][kTerms][4];
-  auto load = [&](int j, int c) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) w[j][t] = ldg128_nt(wp + (size_t)c * 4096 + t * 1024);
-    sw[j] = ldg32_nt(sp + (size_t)c * 256);
-#pragma unroll
-    for (int term = 0; term < kTerms; ++term)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) xv[j][term][r] = ldg128(act(term, c, r));
-  };
-#pragma unroll
-  for (int j = 0; j < kRing; ++j)
-    if (c0 + j < c1) load(j, c0 + j);
-  for (int base = c0; base < c1; base += kRing) {
-#pragma unroll
-    for (int j = 0; j < kRing; ++j) {
-      const int c = base + j;
-      if (c < c1) {
-        chunk_mfma<kTerms>(w[j], sw[j], xv[j], acc);
-        if (c + kRing < c1) load(j, c + kRing);
-      }
-    }
-  }
 }
 
 // One 128-wide K chunk of one gate/up tile against up to 16 tokens: 4 MFMAs, one per word. w = this lane's 16
@@ -221,42 +169,83 @@ __global__ __launch_bounds__(64 * kGuWaves) void bf16_gateup_swiglu_kernel(GateU
   a.hs[(size_t)a.T * I + idx] = (uint16_t)mx::bf16_bits(rest);
 }
 
-// grid (H/64), 256 threads. Row block b holds W2 rows [64b, 64b + 64): tile t's MFMA rows are rows
-// 64b + 16t + 0..15. The I/128 chunks are quartered over the waves.
-__global__ __launch_bounds__(256) void bf16_down_kernel(DownArgs a) {
-  __shared__ float red[4][4][64][4];
-  const int b = blockIdx.x;
+// grid (H / 16 / kDownTiles), 64 kDownWaves threads. A workgroup owns kDownTiles consecutive 16-row tiles of one 64-row
+// group (tile t's MFMA rows are W2 rows 64b + 16t + 0..15) over all of K; the I/128 chunks are shared out over the waves,
+// each wave's in flight together (kDownRing of them), and the waves' sums added in wave order.
+// The launch is bound by its memory round trips, not by its bytes (7.8 MB at 7168 x 2048): us a call (both launches) at
+// 1 / 4 / 16 tokens with 2 tiles x 8 waves 12.5 / 13.4 / 17.4, 4 tiles x 4 waves (two round trips a wave) 12.9-13.7 /
+// 13.4-14.2 / 18.4, 1 tile x 8 waves 14.0 / 14.9 / 21.0, 2 x 4 12.8 / 13.6 / 17.5, 2 x 16 12.4 / 13.4 / 18.8.
+constexpr int kDownTiles = 2, kDownWaves = 8, kDownRing = 2;
+
+__global__ __launch_bounds__(64 * kDownWaves) void bf16_down_kernel(DownArgs a) {
+  __shared__ float4 red[kDownWaves][kDownTiles][64];
+  const int b = blockIdx.x * kDownTiles / 4, t0 = blockIdx.x * kDownTiles % 4;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.H, I = a.I;
   const int chunks = I / 128;
-  const int c0 = chunks * wave / 4, c1 = chunks * (wave + 1) / 4;
+  const int c0 = chunks * wave / kDownWaves, c1 = chunks * (wave + 1) / kDownWaves;
   const int q = lane >> 4, tok = min(lane & 15, a.T - 1);
   const TiledOffsets off = tiled_offsets(H, I);
-  const uint8_t* wp = a.blob + off.dn_w + (size_t)b * chunks * 4096 + 16 * lane;
+  const uint8_t* wp = a.blob + off.dn_w + (size_t)b * chunks * 4096 + 1024 * t0 + 16 * lane;
   const uint8_t* sp = a.blob + off.dn_s + (size_t)b * chunks * 256 + 4 * lane;
   const uint8_t* hrow = reinterpret_cast<const uint8_t*>(a.hs + (size_t)tok * I) + 64 * q;
   const size_t lo = (size_t)a.T * I * 2;   // bytes from the hi term to the lo term
-  auto act = [&](int term, int c, int r) { return hrow + term * lo + (size_t)c * 256 + 16 * r; };
-  v4f acc[4];
+  uint4 w[kDownRing][kDownTiles], xv[kDownRing][2][4];
+  uint32_t sw[kDownRing];
+  auto load = [&](int k, int c) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-  stream_group<2>(wp, sp, c0, c1, act, acc);
+    for (int t = 0; t < kDownTiles; ++t) w[k][t] = ldg128_nt(wp + (size_t)c * 4096 + 1024 * t);
+    sw[k] = ldg32_nt(sp + (size_t)c * 256);
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+    for (int term = 0; term < 2; ++term)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][t][lane][i] = acc[t][i];
+      for (int r = 0; r < 4; ++r) xv[k][term][r] = ldg128(hrow + term * lo + (size_t)c * 256 + 16 * r);
+  };
+  v4f acc[kDownTiles];
+#pragma unroll
+  for (int t = 0; t < kDownTiles; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < kDownRing; ++k)
+    if (c0 + k < c1) load(k, c0 + k);
+  for (int base = c0; base < c1; base += kDownRing) {
+#pragma unroll
+    for (int k = 0; k < kDownRing; ++k) {
+      const int c = base + k;
+      if (c < c1) {
+#pragma unroll
+        for (int t = 0; t < kDownTiles; ++t) {
+          const uint32_t code = (sw[k] >> (8 * (t0 + t))) & 0xFF;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const v8bf m = fp4_word_bf16(word_of(w[k][t], r), code);
+#pragma unroll
+            for (int term = 0; term < 2; ++term)
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, __builtin_bit_cast(v8bf, xv[k][term][r]), acc[t], 0, 0, 0);
+          }
+        }
+        if (c + kDownRing < c1) load(k, c + kDownRing);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < kDownTiles; ++t) red[wave][t][lane] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
   __syncthreads();
-  const int t = tid >> 6, col = lane & 15;
-  if (col < a.T) {
-    uint32_t out[4];
+  const int col = lane & 15;
+  if (wave < kDownTiles && col < a.T) {   // wave t finishes tile t
+    float4 s = red[0][wave][lane];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      out[i] = mx::bf16_bits(((red[0][t][lane][i] + red[1][t][lane][i]) + red[2][t][lane][i]) + red[3][t][lane][i]);
+    for (int v = 1; v < kDownWaves; ++v) {
+      const float4 r = red[v][wave][lane];
+      s.x = s.x + r.x;
+      s.y = s.y + r.y;
+      s.z = s.z + r.z;
+      s.w = s.w + r.w;
+    }
     uint2 packed;
-    packed.x = out[0] | (out[1] << 16);
-    packed.y = out[2] | (out[3] << 16);
-    *reinterpret_cast<uint2*>(a.y + (size_t)col * H + 64 * b + 16 * t + 4 * q) = packed;
+    packed.x = mx::bf16_bits(s.x) | (mx::bf16_bits(s.y) << 16);
+    packed.y = mx::bf16_bits(s.z) | (mx::bf16_bits(s.w) << 16);
+    *reinterpret_cast<uint2*>(a.y + (size_t)col * H + 64 * b + 16 * (t0 + wave) + 4 * q) = packed;
   }
 }
 
@@ -288,7 +277,7 @@ int mx_expert_forward_bf16(mx_ctx* ctx, const void* tiled, int32_t H, int32_t I,
   hipLaunchKernelGGL(bf16_gateup_swiglu_kernel, dim3(I / 8), dim3(64 * kGuWaves), 0, st, ga);
   MX_LAUNCH_CHECK("bf16_gateup_swiglu_kernel");
   DownArgs da{(const uint8_t*)tiled, hs, y, H, I, T};
-  hipLaunchKernelGGL(bf16_down_kernel, dim3(H / 64), dim3(256), 0, st, da);
+  hipLaunchKernelGGL(bf16_down_kernel, dim3(H / 16 / kDownTiles), dim3(64 * kDownWaves), 0, st, da);
   MX_LAUNCH_CHECK("bf16_down_kernel");
   return MX_OK;
 }
