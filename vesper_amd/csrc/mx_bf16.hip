@@ -17,14 +17,13 @@
 //
 // Two launches on the caller's stream:
 //   gate/up + SwiGLU (I/8 tiles, 8 waves each): workgroup j owns gate/up tile j (8 W1 rows and the same 8
-//     W3 rows) over all of K, the waves taking contiguous eighths of the chunks, all tokens in one pass
-//     (MFMA columns); the eight partial tiles are added through LDS in wave order, and the workgroup finishes
+//     W3 rows) over all of K, the waves taking contiguous eighths of the chunks, all tokens in one pass; the eight partial tiles are added through LDS in wave order, and the workgroup finishes
 //     its 8 intermediate positions: h = silu(g) * u (* route weight) in FP32 (optionally written out with g
 //     and u), and h as two BF16 terms hi + lo for the down product (hi = bf16(h), lo = bf16(h - hi): their
 //     sum holds h to about 16 significant bits);
 //   down (H/32 row pairs of tiles, 8 waves): W2 rows against hi and lo (two MFMAs per step), the eight waves'
 //     sums added in wave order and rounded once to BF16.
-// Every sum runs in a fixed order (MFMA chains per wave, then waves), independent of T and of scheduling, so
+// Every sum runs in a fixed order (an MFMA chain per word and wave, words, waves), independent of T and of scheduling, so
 // a token's result does not depend on the batch it runs in.
 #include <algorithm>
 #include <cmath>
@@ -45,7 +44,18 @@ constexpr int kMaxTokens = 16;
 constexpr int kGuWaves = 8;      // gate/up: waves per tile, each a contiguous eighth of K
 constexpr int kMaxHidden = 8192;
 constexpr int kMaxInter = 4096;
-constexpr int kRing = 3;         // chunks of weights (and their activations) in flight per wave
+
+// Up to kFewTokens tokens the MFMA's operands are exchanged: A is the activations, its row 4 t + r word r's K range of
+// token t, so ONE 16-byte load per lane serves the four MFMAs of a chunk, and B is the weights (column n = weight row
+// n). MFMA r multiplies word r; of its D (lane (n, g) register i = activation row 4 g + i = token g, word i) register r
+// is the product wanted and the other three are dropped. With a column per token the four operand loads a chunk and
+// term were 4 KB through the CU's load path beside 1 KB of a tile's weights (8 KB beside 2 in down), whatever the
+// number of tokens. Both forms keep one MFMA chain per word and add the four at the end, so a token's result is the
+// same in either. The 7168 x 2048 expert, us a call at 1 / 3 / 4 / 5 / 16 tokens: 12.0 / 12.1 / 12.4 / 12.3 / 17.4 with a
+// column per token at any count, 9.5 / 9.8 / 9.9 / 12.2 / 17.4 with the exchange (a gate/up ring of 4 chunks; of 8, the
+// whole of a wave's K, 10.0 / - / 10.1). What is left is the two launches' ramps and drains: 23.4 MB take 3.4 us at the
+// rate of a plain read.
+constexpr int kFewTokens = 4;
 
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -83,20 +93,95 @@ __device__ __forceinline__ uint32_t word_of(const uint4 v, int r) {
   return r == 0 ? v.x : r == 1 ? v.y : r == 2 ? v.z : v.w;
 }
 
-// One 128-wide K chunk of one gate/up tile against up to 16 tokens: 4 MFMAs, one per word. w = this lane's 16
-// bytes of the tile, code = its E8M0 code, xv[r] = the tokens' BF16 operand for word r.
-__device__ __forceinline__ void tile_chunk_mfma(const uint4& w, uint32_t code, const uint4 (&xv)[4], v4f& acc) {
+// One 128-wide K chunk of one tile: MFMA r multiplies word r of the lane's 16 weight bytes w (E8M0 code `code`) into
+// acc[r]. xv: the activations, kFew one operand for all four words, else one per word and 16 tokens.
+template <bool kFew>
+__device__ __forceinline__ void tile_chunk_mfma(const uint4& w, uint32_t code, const uint4 (&xv)[kFew ? 1 : 4],
+                                                v4f (&acc)[4]) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4_word_bf16(word_of(w, r), code), __builtin_bit_cast(v8bf, xv[r]),
-                                                  acc, 0, 0, 0);
+  for (int r = 0; r < 4; ++r) {
+    const v8bf m = fp4_word_bf16(word_of(w, r), code);
+    if constexpr (kFew) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xv[0]), m, acc[r], 0, 0, 0);
+    else acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, __builtin_bit_cast(v8bf, xv[r]), acc[r], 0, 0, 0);
+  }
+}
+
+// A wave's sums of a tile, the four words' chains added in word order: lane (n, q) holds weight row n of token q in
+// element 0 (kFew), or weight rows 4 q + 0..3 of token n.
+template <bool kFew>
+struct TileSum {
+  float v[kFew ? 1 : 4];
+};
+
+template <bool kFew>
+__device__ __forceinline__ TileSum<kFew> tile_sum(const v4f (&acc)[4]) {
+  TileSum<kFew> s;
+  if constexpr (kFew) {
+    s.v[0] = ((acc[0][0] + acc[1][1]) + acc[2][2]) + acc[3][3];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s.v[i] = ((acc[0][i] + acc[1][i]) + acc[2][i]) + acc[3][i];
+  }
+  return s;
+}
+
+// Chunks [c0, c1) through a register ring of R: load(k, c) fills slot k, mma(k) multiplies it. kFew: no load is under a
+// branch of its own, those past the end repeat the last chunk -- where paths with and without a load meet, the
+// compiler waits for every load in flight before the next product. For more tokens, whose operand loads fill the load
+// path, the repeated chunks cost more (19.0 us a call against 17.4 at 16 tokens). Reading chunk c0 is safe where the
+// range is empty: it is a chunk of the tile.
+template <int R, bool kFew, typename Load, typename Mma>
+__device__ __forceinline__ void stream_ring(int c0, int c1, Load load, Mma mma) {
+  const int n = c1 - c0;
+  if constexpr (kFew) {
+    const int last = max(n - 1, 0);
+#pragma unroll
+    for (int k = 0; k < R; ++k) load(k, c0 + min(k, last));
+    int i = 0;
+    for (; i + R < n; i += R) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        mma(k);
+        load(k, c0 + min(i + k + R, last));
+        __builtin_amdgcn_sched_barrier(0);   // keeps the refills between the products
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (i + k < n) mma(k);
+  } else {
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (k < n) load(k, c0 + k);
+    for (int i = 0; i < n; i += R) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        if (i + k < n) {
+          mma(k);
+          if (i + k + R < n) load(k, c0 + i + k + R);
+        }
+      }
+    }
+  }
+}
+
+// Where a lane's activation operand of word 0 (kFew: its only one) starts in a token's row, and its token.
+template <bool kFew>
+__device__ __forceinline__ int operand_token(int lane, int T) {
+  return min(kFew ? (lane & 15) >> 2 : lane & 15, T - 1);
+}
+template <bool kFew>
+__device__ __forceinline__ int operand_offset(int lane) {
+  return 64 * (lane >> 4) + (kFew ? 16 * (lane & 3) : 0);
 }
 
 // grid (I/8), 64 kGuWaves threads. Tile j = 4 g + t of row group g: MFMA rows 0-7 are W1 rows 8j + 0..7, rows
 // 8-15 the same W3 rows; chunk c of the tile at (g C + c) 4096 + 1024 t, its codes byte t of the chunk's scale
 // words. Wave w streams chunks [C w / 8, C (w + 1) / 8) through a register ring.
+template <bool kFew>
 __global__ __launch_bounds__(64 * kGuWaves) void bf16_gateup_swiglu_kernel(GateUpArgs a) {
-  __shared__ float4 red[kGuWaves][64];
+  constexpr int kRing = kFew ? 4 : 3, kX = kFew ? 1 : 4;
+  __shared__ TileSum<kFew> red[kGuWaves][64];
   __shared__ float tile[16][kMaxTokens + 1];
   const int j = blockIdx.x, g = j >> 2, t = j & 3;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -104,51 +189,37 @@ __global__ __launch_bounds__(64 * kGuWaves) void bf16_gateup_swiglu_kernel(GateU
   const int H = a.H, I = a.I;
   const int chunks = H / 128;
   const int c0 = chunks * wave / kGuWaves, c1 = chunks * (wave + 1) / kGuWaves;
-  const int q = lane >> 4, tok = min(lane & 15, a.T - 1);
+  const int q = lane >> 4, tok = operand_token<kFew>(lane, a.T);
   const uint8_t* wp = a.blob + (size_t)g * chunks * 4096 + t * 1024 + 16 * lane;
   const uint8_t* sp = a.blob + tiled_offsets(H, I).gu_s + (size_t)g * chunks * 256 + 4 * lane;
-  const uint8_t* xrow = reinterpret_cast<const uint8_t*>(a.x + (size_t)tok * H) + 64 * q;
+  const uint8_t* xrow = reinterpret_cast<const uint8_t*>(a.x + (size_t)tok * H) + operand_offset<kFew>(lane);
   uint4 w[kRing];
   uint32_t sw[kRing];
-  uint4 xv[kRing][4];
+  uint4 xv[kRing][kX];
   auto load = [&](int k, int c) {
     w[k] = ldg128_nt(wp + (size_t)c * 4096);
     sw[k] = ldg32_nt(sp + (size_t)c * 256);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) xv[k][r] = ldg128(xrow + (size_t)c * 256 + 16 * r);
+    for (int r = 0; r < kX; ++r) xv[k][r] = ldg128(xrow + (size_t)c * 256 + 16 * r);
   };
-  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+  v4f acc[4];
 #pragma unroll
-  for (int k = 0; k < kRing; ++k)
-    if (c0 + k < c1) load(k, c0 + k);
-  for (int base = c0; base < c1; base += kRing) {
-#pragma unroll
-    for (int k = 0; k < kRing; ++k) {
-      const int c = base + k;
-      if (c < c1) {
-        tile_chunk_mfma(w[k], (sw[k] >> (8 * t)) & 0xFF, xv[k], acc);
-        if (c + kRing < c1) load(k, c + kRing);
-      }
-    }
-  }
-  red[wave][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  for (int r = 0; r < 4; ++r) acc[r] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](int k) { tile_chunk_mfma<kFew>(w[k], (sw[k] >> (8 * t)) & 0xFF, xv[k], acc); };
+  stream_ring<kRing, kFew>(c0, c1, load, mma);
+  red[wave][lane] = tile_sum<kFew>(acc);
   __syncthreads();
   if (wave == 0) {
-    // lane l holds MFMA rows 4 (l / 16) + 0..3 of token column l % 16; the waves' tiles added in wave order
-    float4 s = red[0][lane];
+    // the waves' tiles added in wave order
+    TileSum<kFew> s = red[0][lane];
+    const int n = lane & 15;
 #pragma unroll
-    for (int v = 1; v < kGuWaves; ++v) {
-      const float4 r = red[v][lane];
-      s.x = s.x + r.x;
-      s.y = s.y + r.y;
-      s.z = s.z + r.z;
-      s.w = s.w + r.w;
+    for (int i = 0; i < kX; ++i) {
+#pragma unroll
+      for (int v = 1; v < kGuWaves; ++v) s.v[i] = s.v[i] + red[v][lane].v[i];
+      if constexpr (kFew) tile[n][q] = s.v[i];
+      else tile[4 * q + i][n] = s.v[i];
     }
-    const int col = lane & 15;
-    tile[4 * q + 0][col] = s.x;
-    tile[4 * q + 1][col] = s.y;
-    tile[4 * q + 2][col] = s.z;
-    tile[4 * q + 3][col] = s.w;
   }
   __syncthreads();
   // thread (token, i): intermediate position 8 j + i, gate row i and up row 8 + i of the tile
@@ -172,26 +243,28 @@ __global__ __launch_bounds__(64 * kGuWaves) void bf16_gateup_swiglu_kernel(GateU
 // grid (H / 16 / kDownTiles), 64 kDownWaves threads. A workgroup owns kDownTiles consecutive 16-row tiles of one 64-row
 // group (tile t's MFMA rows are W2 rows 64b + 16t + 0..15) over all of K; the I/128 chunks are shared out over the waves,
 // each wave's in flight together (kDownRing of them), and the waves' sums added in wave order.
-// The launch is bound by its memory round trips, not by its bytes (7.8 MB at 7168 x 2048): us a call (both launches) at
-// 1 / 4 / 16 tokens with 2 tiles x 8 waves 12.5 / 13.4 / 17.4, 4 tiles x 4 waves (two round trips a wave) 12.9-13.7 /
+// The launch is bound by its memory round trips, not by its bytes (7.8 MB at 7168 x 2048): us a call (both launches, a
+// column per token at any count) at 1 / 4 / 16 tokens with 2 tiles x 8 waves 12.5 / 13.4 / 17.4, 4 tiles x 4 waves (two round trips a wave) 12.9-13.7 /
 // 13.4-14.2 / 18.4, 1 tile x 8 waves 14.0 / 14.9 / 21.0, 2 x 4 12.8 / 13.6 / 17.5, 2 x 16 12.4 / 13.4 / 18.8.
 constexpr int kDownTiles = 2, kDownWaves = 8, kDownRing = 2;
 
+template <bool kFew>
 __global__ __launch_bounds__(64 * kDownWaves) void bf16_down_kernel(DownArgs a) {
-  __shared__ float4 red[kDownWaves][kDownTiles][64];
+  constexpr int kX = kFew ? 1 : 4;
+  __shared__ TileSum<kFew> red[kDownWaves][kDownTiles][64];
   const int b = blockIdx.x * kDownTiles / 4, t0 = blockIdx.x * kDownTiles % 4;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.H, I = a.I;
   const int chunks = I / 128;
   const int c0 = chunks * wave / kDownWaves, c1 = chunks * (wave + 1) / kDownWaves;
-  const int q = lane >> 4, tok = min(lane & 15, a.T - 1);
+  const int q = lane >> 4, tok = operand_token<kFew>(lane, a.T);
   const TiledOffsets off = tiled_offsets(H, I);
   const uint8_t* wp = a.blob + off.dn_w + (size_t)b * chunks * 4096 + 1024 * t0 + 16 * lane;
   const uint8_t* sp = a.blob + off.dn_s + (size_t)b * chunks * 256 + 4 * lane;
-  const uint8_t* hrow = reinterpret_cast<const uint8_t*>(a.hs + (size_t)tok * I) + 64 * q;
+  const uint8_t* hrow = reinterpret_cast<const uint8_t*>(a.hs + (size_t)tok * I) + operand_offset<kFew>(lane);
   const size_t lo = (size_t)a.T * I * 2;   // bytes from the hi term to the lo term
-  uint4 w[kDownRing][kDownTiles], xv[kDownRing][2][4];
+  uint4 w[kDownRing][kDownTiles], xv[kDownRing][2][kX];
   uint32_t sw[kDownRing];
   auto load = [&](int k, int c) {
 #pragma unroll
@@ -200,52 +273,40 @@ __global__ __launch_bounds__(64 * kDownWaves) void bf16_down_kernel(DownArgs a) 
 #pragma unroll
     for (int term = 0; term < 2; ++term)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) xv[k][term][r] = ldg128(hrow + term * lo + (size_t)c * 256 + 16 * r);
+      for (int r = 0; r < kX; ++r) xv[k][term][r] = ldg128(hrow + term * lo + (size_t)c * 256 + 16 * r);
   };
-  v4f acc[kDownTiles];
+  v4f acc[kDownTiles][4];
 #pragma unroll
-  for (int t = 0; t < kDownTiles; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < kDownTiles; ++t)
 #pragma unroll
-  for (int k = 0; k < kDownRing; ++k)
-    if (c0 + k < c1) load(k, c0 + k);
-  for (int base = c0; base < c1; base += kDownRing) {
+    for (int r = 0; r < 4; ++r) acc[t][r] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](int k) {
 #pragma unroll
-    for (int k = 0; k < kDownRing; ++k) {
-      const int c = base + k;
-      if (c < c1) {
+    for (int t = 0; t < kDownTiles; ++t)
 #pragma unroll
-        for (int t = 0; t < kDownTiles; ++t) {
-          const uint32_t code = (sw[k] >> (8 * (t0 + t))) & 0xFF;
+      for (int term = 0; term < 2; ++term)
+        tile_chunk_mfma<kFew>(w[k][t], (sw[k] >> (8 * (t0 + t))) & 0xFF, xv[k][term], acc[t]);
+  };
+  stream_ring<kDownRing, kFew>(c0, c1, load, mma);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const v8bf m = fp4_word_bf16(word_of(w[k][t], r), code);
-#pragma unroll
-            for (int term = 0; term < 2; ++term)
-              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, __builtin_bit_cast(v8bf, xv[k][term][r]), acc[t], 0, 0, 0);
-          }
-        }
-        if (c + kDownRing < c1) load(k, c + kDownRing);
-      }
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < kDownTiles; ++t) red[wave][t][lane] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+  for (int t = 0; t < kDownTiles; ++t) red[wave][t][lane] = tile_sum<kFew>(acc[t]);
   __syncthreads();
-  const int col = lane & 15;
-  if (wave < kDownTiles && col < a.T) {   // wave t finishes tile t
-    float4 s = red[0][wave][lane];
+  const int n = lane & 15;
+  if (wave < kDownTiles && (kFew ? q : n) < a.T) {   // wave t finishes tile t
+    TileSum<kFew> s = red[0][wave][lane];
 #pragma unroll
-    for (int v = 1; v < kDownWaves; ++v) {
-      const float4 r = red[v][wave][lane];
-      s.x = s.x + r.x;
-      s.y = s.y + r.y;
-      s.z = s.z + r.z;
-      s.w = s.w + r.w;
+    for (int i = 0; i < kX; ++i)
+#pragma unroll
+      for (int v = 1; v < kDownWaves; ++v) s.v[i] = s.v[i] + red[v][wave][lane].v[i];
+    uint16_t* y = a.y + (size_t)(kFew ? q : n) * H + 64 * b + 16 * (t0 + wave);
+    if constexpr (kFew) {
+      y[n] = (uint16_t)mx::bf16_bits(s.v[0]);
+    } else {
+      uint2 packed;
+      packed.x = mx::bf16_bits(s.v[0]) | (mx::bf16_bits(s.v[1]) << 16);
+      packed.y = mx::bf16_bits(s.v[2]) | (mx::bf16_bits(s.v[3]) << 16);
+      *reinterpret_cast<uint2*>(y + 4 * q) = packed;
     }
-    uint2 packed;
-    packed.x = mx::bf16_bits(s.x) | (mx::bf16_bits(s.y) << 16);
-    packed.y = mx::bf16_bits(s.z) | (mx::bf16_bits(s.w) << 16);
-    *reinterpret_cast<uint2*>(a.y + (size_t)col * H + 64 * b + 16 * (t0 + wave) + 4 * q) = packed;
   }
 }
 
@@ -274,10 +335,11 @@ int mx_expert_forward_bf16(mx_ctx* ctx, const void* tiled, int32_t H, int32_t I,
   if (int s = mxi::scratch(ctx, bf16_scratch_bytes(I, T), &base)) return s;
   uint16_t* hs = (uint16_t*)base;
   GateUpArgs ga{(const uint8_t*)tiled, x, route_w, h, gu, hs, H, I, T};
-  hipLaunchKernelGGL(bf16_gateup_swiglu_kernel, dim3(I / 8), dim3(64 * kGuWaves), 0, st, ga);
+  const bool few = T <= kFewTokens;
+  hipLaunchKernelGGL(few ? bf16_gateup_swiglu_kernel<true> : bf16_gateup_swiglu_kernel<false>, dim3(I / 8), dim3(64 * kGuWaves), 0, st, ga);
   MX_LAUNCH_CHECK("bf16_gateup_swiglu_kernel");
   DownArgs da{(const uint8_t*)tiled, hs, y, H, I, T};
-  hipLaunchKernelGGL(bf16_down_kernel, dim3(H / 16 / kDownTiles), dim3(64 * kDownWaves), 0, st, da);
+  hipLaunchKernelGGL(few ? bf16_down_kernel<true> : bf16_down_kernel<false>, dim3(H / 16 / kDownTiles), dim3(64 * kDownWaves), 0, st, da);
   MX_LAUNCH_CHECK("bf16_down_kernel");
   return MX_OK;
 }
