@@ -10,15 +10,16 @@
 // checked on gfx950 for every code and value, code 255 giving NaN as the format defines).
 //
 // MFMA mapping (measured on gfx950): A lane l = row l % 16, K 8 (l / 16) + 0..7; B lane l = column l % 16,
-// same K; D lane l register i = row 4 (l / 16) + i, column l % 16. A is 16 weight rows, B is up to 16 tokens.
+// same K; D lane l register i = row 4 (l / 16) + i, column l % 16. A is 16 weight rows, B is up to 16 tokens (exchanged
+// for few tokens: kFewTokens).
 // In the tiled layout a lane (m, q) of tile t holds the 32 E2M1 values of row m, K block 4c + q as four
 // 32-bit words; MFMA r of chunk c takes word r of every lane, i.e. K = 32 (4c + q) + 8r + 0..7 at lane group
 // q, and the activations are read with the same map, so every product pairs the right operands.
 //
 // Two launches on the caller's stream:
 //   gate/up + SwiGLU (I/8 tiles, 8 waves each): workgroup j owns gate/up tile j (8 W1 rows and the same 8
-//     W3 rows) over all of K, the waves taking contiguous eighths of the chunks, all tokens in one pass; the eight partial tiles are added through LDS in wave order, and the workgroup finishes
-//     its 8 intermediate positions: h = silu(g) * u (* route weight) in FP32 (optionally written out with g
+//     W3 rows) over all of K, the waves taking contiguous eighths of the chunks, all tokens in one
+//     pass; the eight partial tiles are added through LDS in wave order, and the workgroup finishes its 8 intermediate positions: h = silu(g) * u (* route weight) in FP32 (optionally written out with g
 //     and u), and h as two BF16 terms hi + lo for the down product (hi = bf16(h), lo = bf16(h - hi): their
 //     sum holds h to about 16 significant bits);
 //   down (H/32 row pairs of tiles, 8 waves): W2 rows against hi and lo (two MFMAs per step), the eight waves'
