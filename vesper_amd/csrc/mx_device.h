@@ -70,12 +70,15 @@ __device__ __forceinline__ void global_to_lds4(const void* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds) : "m0");
 }
 
-// Workgroup barrier for the global->LDS copy pipelines: the caller has already waited for its own copies
-// and LDS reads (s_waitcnt) as far as the barrier must cover. Even the local-only fences of lds_barrier
-// would wait for every copy in flight (the copies write LDS), so the barrier is issued bare; the empty
-// assembly statements with a memory clobber keep the compiler from moving memory operations across it.
+// Workgroup barrier for the global->LDS copy pipelines: past it, a copy may overwrite the stage this wave has just
+// read, so the wave's LDS reads have to have returned -- waited for here (lgkmcnt(0)), not left to where the compiler
+// happens to place the products that use them. Copies are the caller's: it has waited for its own (s_waitcnt) as far as
+// the barrier must cover. Even the local-only fences of lds_barrier would wait for every copy in flight (the copies
+// write LDS), so the barrier is issued bare; the empty assembly statements with a memory clobber keep the compiler
+// from moving memory operations across it.
 __device__ __forceinline__ void copy_barrier() {
   asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }

@@ -382,7 +382,6 @@ __global__ __launch_bounds__(kGThreads) void grouped_down_kernel(GemmArgs a) {
           asm volatile("" : "+v"(acc[0][u]), "+v"(acc[1][u]), "+v"(acc[2][u]), "+v"(acc[3][u]));
         }
       }
-      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave's reads of chunk c are done
       copy_barrier();
     }
   }
