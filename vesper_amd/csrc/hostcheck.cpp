@@ -1,9 +1,10 @@
-// Host build of the device numerics (mx_numerics.h) for exhaustive CPU comparison with the oracle.
-// Nothing here runs on the GPU path; libmxmoe.so compiles the same header for gfx950.
+// Host build of the device numerics (mx_numerics.h) for exhaustive CPU comparison with the oracle, and of the prefill
+// ring's layout (mx_ring.h). Nothing here runs on the GPU path; libmxmoe.so compiles the same headers for gfx950.
 #include <cmath>
 #include <cstdint>
 
 #include "mx_numerics.h"
+#include "mx_ring.h"
 
 extern "C" {
 
@@ -79,6 +80,16 @@ int64_t mxh_act128_quotient_check(int64_t* code_mismatches, float* max_quotient,
   *max_quotient = qmax;
   *pairs = n;
   return bad;
+}
+
+// Prefill gate/up ring with `live` token tiles: bytes of a stage, stages, bytes of the LDS, where a stage's activations
+// start, and the token tiles that a read from tile u takes.
+void mxh_prefill_ring(int32_t live, int32_t u, int32_t* out) {
+  out[0] = mxring::xstage_bytes(live);
+  out[1] = mxring::xstages(live);
+  out[2] = mxring::kXLdsBytes;
+  out[3] = mxring::kXStageB;
+  out[4] = mxring::xacts_read(live, u);
 }
 
 }  // extern "C"

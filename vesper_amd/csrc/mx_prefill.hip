@@ -24,6 +24,7 @@
 #include "mx_device.h"
 #include "mx_internal.h"
 #include "mx_numerics.h"
+#include "mx_ring.h"
 
 namespace {
 
@@ -447,17 +448,7 @@ __global__ __launch_bounds__(kGThreads) void grouped_down_kernel(GemmArgs a) {
 // not see writing LDS, so it places no wait for them before a read -- the wave's own vmcnt wait and the
 // barrier at the top of each step order them.
 constexpr int kXThreads = 512;
-// a stage: the 8 groups' weight tiles (group w, tile t at 1 KB x (4 w + t)), their scale words (256 B per
-// group), then the activations of the tile's live token tiles: token tile u, block b at 1 KB x (4 u + b)
-constexpr int kXStageA = 0, kXStageAS = 32768, kXStageB = 34816;
-constexpr int xstage_bytes(int live) { return kXStageB + 4096 * live; }
-// stages in the ring with `live` token tiles: as many as the LDS holds, at most 4
-constexpr int xstages(int live) { return 160 * 1024 / xstage_bytes(live) < 4 ? 160 * 1024 / xstage_bytes(live) : 4; }
-constexpr int xlds_bytes(int live) { return xstages(live) * xstage_bytes(live); }
-constexpr int xlds_max(int live = 8) {
-  return live == 0 ? 0 : xlds_bytes(live) > xlds_max(live - 1) ? xlds_bytes(live) : xlds_max(live - 1);
-}
-constexpr int kXLdsBytes = xlds_max();
+using namespace mxring;
 static_assert(xstages(8) >= 2 && kXLdsBytes <= 160 * 1024 && 2 * kTileRows * kEpiRowG * 2 <= kXLdsBytes,
               "exact gate/up LDS layout");
 
@@ -502,15 +493,14 @@ __device__ __forceinline__ void lds_read_weights(uint32_t a_addr, uint32_t s_add
   for (int b = 0; b < 4; ++b) sw[b] = ps[16 * b];
 }
 
-// four token tiles' activation operands of one block: 16 bytes at addr + 4 KB j, j < 4. Plain LDS loads, so
-// that token tile j's MFMAs wait only for its own read (lgkmcnt(3 - j)) instead of all four (2.5 % slower
-// per prefill with a single wait).
-__device__ __forceinline__ void lds_read_acts4(uint32_t addr, mxd::u32x4_t (&x)[4]) {
+// up to four token tiles' activation operands of one block: 16 bytes at addr + 4 KB j, j < count (a constant once the
+// loops are unrolled). Plain LDS loads, so that token tile j's MFMAs wait only for its own read (lgkmcnt(3 - j))
+// instead of all four (2.5 % slower per prefill with a single wait).
+__device__ __forceinline__ void lds_read_acts(uint32_t addr, int count, mxd::u32x4_t (&x)[4]) {
   const lds_u32x4_ptr p = (lds_u32x4_ptr)(size_t)addr;
-  x[0] = p[0];
-  x[1] = p[256];
-  x[2] = p[512];
-  x[3] = p[768];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (j < count) x[j] = p[256 * j];
 }
 
 // One wave's copies and LDS operand addresses (see gateup_exact_kernel).
@@ -588,7 +578,7 @@ __device__ __forceinline__ void exact_stream(const ExactStream& s, v4f (&acc)[4]
 #pragma unroll
       for (int u = 0; u <= L; ++u) {
         if (u < L) {
-          if ((u & 3) == 0) lds_read_acts4(s.lb + so + (4 * u + b) * 1024, x);
+          if ((u & 3) == 0) lds_read_acts(s.lb + so + (4 * u + b) * 1024, xacts_read(L, u), x);
           mxd::u32x4_t xw = x[u & 3];
           asm volatile("" : "+v"(xw));
           const v8bf xv = __builtin_bit_cast(v8bf, xw);
