@@ -301,7 +301,8 @@ int mx_act_quant128(mx_ctx* ctx, const uint16_t* x_bf16, uint8_t* q, float* s, i
                     void* stream);
 /* y[T][N] (BF16) = projection of x[T][H=K] (BF16): quantize with the block's activation quantizer, then the
  * block-scaled product. Optional outputs: trace [T][N] FP32 sums, q_out [T][K] codes, s_out scales
- * ([T][K/32] E8M0 or [T][K/128] FP32) -- the stage dict of projections.py:146-154. */
+ * ([T][K/32] E8M0 or [T][K/128] FP32) -- the stage dict of projections.py:146-154. y and trace may share bytes
+ * with x: the call reads x before it writes them. */
 int mx_fp8_projection(mx_ctx* ctx, const void* tiled, int32_t n, int32_t k, int32_t block, const uint16_t* x_bf16,
                       int32_t tokens, uint16_t* y_bf16, float* trace, uint8_t* q_out, void* s_out, void* stream);
 
@@ -317,7 +318,8 @@ int mx_fp8_grouped_projection(mx_ctx* ctx, const void* tiled, int32_t groups, in
 /* FP8 block-32 expert (the shared expert's format, src/vesper/shared.py:20-24,141-170 with
  * gemv_fp8_shared, shared_probe.cu:4-49): the MXFP4 expert's stage sequence with E4M3 weights and E8M0
  * scales per 32 x 32 block. w1/w3/w2 are tiled blobs (mx_fp8_tile, block 32) of W1 [I][H], W3 [I][H] and
- * W2 [H][I]; route_w NULL = unweighted. Same stage buffers and semantics as mx_expert_forward. */
+ * W2 [H][I]; route_w NULL = unweighted. Same stage buffers and semantics as mx_expert_forward; y and the stages
+ * may share bytes with x. */
 int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1_tiled, const void* w3_tiled, const void* w2_tiled,
                           int32_t hidden, int32_t intermediate, const uint16_t* x_bf16, int32_t tokens,
                           float swiglu_limit, const float* route_w, uint16_t* y_bf16,

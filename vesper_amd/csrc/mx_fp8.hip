@@ -490,9 +490,9 @@ __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
       const uint32_t b1 = mx::bf16_bits(pair[0][pt][row]), b3 = mx::bf16_bits(pair[1][pt][row]);
       const float v = mxd::swiglu_element(b1, b3, a.limit, a.route_w != nullptr, a.route_w ? a.route_w[tok0 + pt] : 1.f,
                                           a.swiglu_trace ? a.swiglu_trace + o * 5 : nullptr);
-      a.din[o] = (uint16_t)mx::bf16_bits(v);
       if (a.y) a.y[o] = (uint16_t)b1;
       if (a.y3) a.y3[o] = (uint16_t)b3;
+      a.din[o] = (uint16_t)mx::bf16_bits(v);   // last: a caller may keep it where W1's or W3's output was
     }
     return;
   }
@@ -791,6 +791,13 @@ void launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st
   else if (sh.W == 16 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 16, 2, 1>(a, P, st);
 }
 
+// Whether a[0 .. na) and b[0 .. nb) share bytes (a null pointer shares none). A launch that quantizes its own input
+// reads it while other workgroups already write their outputs: where the two share bytes (a projection in place, a down
+// input kept in y), a quantizer launch of its own reads it first.
+bool overlap(const void* a, uint64_t na, const void* b, uint64_t nb) {
+  return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 // Whether the GEMV quantizes a plain call's activations itself (fp8_row_gemv_kernel, few tokens).
 bool fp8_fused_ok(int N, int K, int T) { return T <= kFusedMaxTokens && fp8_fused_passes(fp8_row_shape(N, K, T), K, T) > 0; }
 
@@ -915,7 +922,9 @@ int mx_fp8_projection(mx_ctx* ctx, const void* tiled, int32_t N, int32_t K, int3
   void* sc = s_out ? s_out : (void*)((uint8_t*)base + q_b);
   MX_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)sc & 3) == 0, "mx_fp8_projection: q 16-byte, s 4-byte aligned");
   float* partial = (float*)((uint8_t*)base + q_b + s_b);
-  if (!q_out && !s_out && fp8_fused_ok(N, K, T))   // the GEMV quantizes x itself
+  const uint64_t x_b = (uint64_t)T * K * 2, y_b = (uint64_t)T * N * 2;
+  if (!q_out && !s_out && fp8_fused_ok(N, K, T) && !overlap(x, x_b, y, y_b) &&
+      !overlap(x, x_b, trace, 2 * y_b))   // the GEMV quantizes x itself
     return launch_fp8_product((const uint8_t*)tiled, N, K, block, nullptr, nullptr, T, y, trace, partial, st, x);
   if (ordered) {
     if (int s = launch_quant_ordered(block, x, q, sc, T, K, st)) return s;
@@ -996,10 +1005,14 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
                  ((uintptr_t)a.y3 & 7) == 0 && ((uintptr_t)din & 3) == 0 && ((uintptr_t)s & 3) == 0 &&
                  ((uintptr_t)ds & 3) == 0,
              "stage buffers: q/down_q 16-byte, w1/w3 8-byte, scales and down_input 4-byte aligned");
-  // few tokens: each launch quantizes its own input, unless the caller asks for those codes (or, for the down
-  // input, gives a buffer that 16-byte loads cannot read); more tokens: codes in the GEMV's load order
+  // few tokens: each launch quantizes its own input, unless the caller asks for those codes or gives an output that
+  // shares bytes with it (or, for the down input, a buffer that 16-byte loads cannot read); more tokens: codes in the
+  // GEMV's load order
+  const uint64_t xh = (uint64_t)T * H * 2, xi = (uint64_t)T * I * 2;   // bytes of [T][H] and of [T][I]
   const bool own_q = !stages || (!stages->q && !stages->s);
-  const int p1 = own_q ? fp8_fused_passes(kPairShape, H, T) : 0;
+  const bool shared_x = overlap(x, xh, din, xi) || overlap(x, xh, a.y, xi) || overlap(x, xh, a.y3, xi) ||
+                        overlap(x, xh, a.swiglu_trace, 10 * xi);   // 5 floats an element
+  const int p1 = own_q && !shared_x ? fp8_fused_passes(kPairShape, H, T) : 0;
   a.ordered = own_q;
   if (p1) a.x = x;
   else if (int e = own_q ? launch_quant_ordered(32, x, q, s, T, H, st) : mx_act_quant32(ctx, x, q, s, T, H, stream))
@@ -1007,7 +1020,7 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
   launch_row_gemv<32, kPairShape.W, 1, 2, true>(a, p1, st);
   MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
   const bool own_dq = (!stages || (!stages->down_q && !stages->down_s)) && ((uintptr_t)din & 15) == 0;
-  if (own_dq && fp8_fused_ok(H, I, T))
+  if (own_dq && fp8_fused_ok(H, I, T) && !overlap(din, xi, y, xh))
     return launch_fp8_product((const uint8_t*)w2, H, I, 32, nullptr, nullptr, T, y, nullptr, nullptr, st, din);
   if (int e = own_dq ? launch_quant_ordered(32, din, dq, ds, T, I, st) : mx_act_quant32(ctx, din, dq, ds, T, I, stream))
     return e;
