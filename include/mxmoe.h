@@ -10,8 +10,8 @@
  * The reference binds CUDA probe kernels through ctypes (src/vesper/cuda.py);
  * each declaration below names the reference interface it replaces.
  *
- * A context keeps a small reusable device buffer (scratch), and a layer
- * keeps its per-call buffers: calls on one context, or on one layer, must not
+ * A context keeps a reusable device buffer (scratch, 4 MiB from mx_create on,
+ * grown by calls that need more), and a layer keeps its per-call buffers: calls on one context, or on one layer, must not
  * run concurrently on different streams. Use one context per stream that runs
  * alongside others, as the reference serialises calls per Device
  * (src/vesper/connected.py:131-133).

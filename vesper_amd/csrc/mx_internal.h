@@ -18,9 +18,14 @@ struct mx_ctx {
   std::mutex lock;
   std::unordered_map<void*, uint64_t> owned;        // device allocations
   std::unordered_map<void*, uint64_t> pinned;       // host pinned allocations
-  void* scratch = nullptr;                          // small reusable device scratch
+  void* scratch = nullptr;                          // reusable device scratch, MX_SCRATCH_START bytes or more
   uint64_t scratch_bytes = 0;
 };
+
+// The scratch a context starts with. Growing it frees and allocates, which synchronises the device and fails under
+// stream capture; an FP8 call of up to 32 tokens over widths up to 100,000 (codes and scales in whole tiles of 16
+// tokens: 32 x width x 33 / 32 bytes) and an FP8 or BF16 expert call fit from the start.
+#define MX_SCRATCH_START (4u << 20)
 
 // By-value kernel argument of mx_layer_set_experts: up to 64 table entries per launch.
 #define MX_EXPERT_BATCH 64

@@ -70,9 +70,13 @@ int mx_create(int device, uint64_t cap_bytes, mx_ctx** out) {
   MX_HIP(hipSetDevice(device));
   MX_HIP(hipFree(nullptr));  // initialise the device's primary context now
   if (int s = noalloc_scratch_init(device)) return s;
+  void* scratch = nullptr;
+  MX_HIP(hipMalloc(&scratch, MX_SCRATCH_START));
   mx_ctx* ctx = new mx_ctx();
   ctx->device = device;
   ctx->cap = cap_bytes;
+  ctx->scratch = scratch;
+  ctx->scratch_bytes = MX_SCRATCH_START;
   *out = ctx;
   return MX_OK;
 }
