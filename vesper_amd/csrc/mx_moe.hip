@@ -1286,11 +1286,21 @@ __global__ __launch_bounds__(256) void router_tile_kernel(RouterArgs a) {
   }
 }
 
-// The router's logits (and scores and selection values) of T tokens, by either kernel with the same bits. us at 17 / 24
-// / 32 / 64 / 333 tokens: 256 experts x 7168 9.8 / 10.0 / 11.9 / 19.8 / 81 with an expert a workgroup, 10.4 / 10.3 / 10.5 /
-// 10.9 / 29.5 with 8 x 8 tiles; 384 x 5120 10.1 / 10.8 / 12.7 / 22.1 / 91 and 8.6 / 8.6 / 8.8 / 10.3 / 28.9.
+// Whether the tiles take a router call: from 25 tokens, where they are enough work to share. A tile's thread walks all of
+// H for 64 sums, so few tiles of a wide router wait longer than an expert a workgroup does. us with an expert a workgroup
+// / tiles, 7168 wide: 256 experts x 25 tokens (6400 sums) 10.8 / 12.1, 128 x 32 (4096) 9.6 / 12.1, 64 x 64 (4096) 9.7 /
+// 10.6, 256 x 32 (8192) 12.7 / 12.1, 64 x 128 (8192) 12.2 / 10.9, 32 x 333 16.9 / 11.7, 384 x 25 14.9 / 11.9, 256 x 333
+// 75 / 29; 8192 wide the same line (64 x 48 9.7 / 11.5, 64 x 128 13.4 / 12.1). Up to 5120 wide the tiles are even or
+// better at every count (128 x 25 8.8 / 8.6, 256 x 25 9.7 / 9.9, 8 x 64 8.9 / 8.7; 1024 wide 256 x 25 8.7 / 5.4). The
+// tiles are one grid dimension, which holds 2^24 - 1 workgroups of 256 threads.
+bool router_tiles(int T, int E, int H) {
+  const int64_t tiles = (((int64_t)E + kRouterTile - 1) / kRouterTile) * (((int64_t)T + kRouterTile - 1) / kRouterTile);
+  return T > 24 && (H <= 5120 || (int64_t)E * T >= 8192) && tiles < (1 << 24);
+}
+
+// The router's logits (and scores and selection values) of T tokens, by either kernel with the same bits.
 int launch_router(const RouterArgs& r, hipStream_t st) {
-  if (r.T > 24)
+  if (router_tiles(r.T, r.E, r.H))
     hipLaunchKernelGGL(router_tile_kernel,
                        dim3((unsigned)((r.E + kRouterTile - 1) / kRouterTile) * (unsigned)((r.T + kRouterTile - 1) / kRouterTile)),
                        dim3(256), 0, st, r);
