@@ -195,7 +195,7 @@ struct Fp8Args {
   const void* xs;      // block 32: uint8 [T][K/32]; block 128: float [T][K/128]
   uint16_t* y;         // [T][N] BF16
   float* trace;        // [T][N] FP32 sums, nullable
-  float* partial;      // split-K GEMM: [splits][T][N] FP32 partial sums (written instead of y)
+  float* partial;      // split K: [splits][T][N] FP32 partial sums (written instead of y)
   const uint16_t* x;   // fused GEMV (few tokens): the BF16 input [T][K], quantized in the kernel
   int ordered;         // GEMV: xq and xs as fp8_quant_ordered_kernel writes them, else [T][K] rows
   int64_t x_stride;    // activation elements per token: K, or groups x K when grouped
@@ -214,8 +214,8 @@ struct Fp8Args {
 // consecutive tiles over all of K: wave w takes set w % M and the (w / M)-th of W / M contiguous K parts, streams its
 // chunks (2 KB of weights per tile and chunk, non-temporal loads, each chunk's activation operands loaded once for its
 // TM tiles) through a register ring of row_ring chunks, and the K parts' partial tiles are added through LDS in
-// K-part order. No K range is shared between workgroups, so no partial sums leave the workgroup: no
-// handoff, no reduce launch.
+// K-part order. K is shared between workgroups only where few rows and a long K would leave most of the chip
+// idle (RowShape::S): elsewhere no partial sums leave the workgroup and there is no reduce launch.
 // Bound by the weight stream and, for several tokens, by the requests that the activations add to it: a chunk's codes
 // of 16 tokens as row pieces were 32 requests and their scales 16, beside 16 for a tile's weights, so a wave takes two
 // tiles where there are enough and the codes come in load order (fp8_quant_ordered_kernel). 16 tokens, us a call:
@@ -311,7 +311,8 @@ __device__ __forceinline__ void row_mma(const RowChunk<TM, NT>& r, v4f (&acc)[NT
   }
 }
 
-// grid (ceil(tile sets / M), ceil(T / (16 NT))), 64 W threads.
+// grid (ceil(tile sets / M), ceil(T / (16 NT)), K splits), 64 W threads. With more than one split a workgroup writes its
+// FP32 sums to a.partial (fp8_splitk_reduce_kernel adds them in split order).
 template <int kBlock, bool kFused, int W, int M, int TM, int NT, int P, bool kPair>
 __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
   static_assert(W % M == 0 && 4 * P * M <= kTileQRows && M * TM * NT <= W && (NT == 1 || !kFused) &&
@@ -358,7 +359,13 @@ __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
   src.x_chunk = a.ordered ? 2048 : 128;
   src.x_half = a.ordered ? 1024 : 64;
   src.xs_chunk = a.ordered ? 64 : 4;
-  const int c0 = (C * kp) / KP, n = (C * (kp + 1)) / KP - c0;
+  // the workgroup's chunks: all of K, or its share of them (blockIdx.z of gridDim.z)
+  int cb = 0, cw = C;
+  if (gridDim.z > 1) {
+    cb = (int)((int64_t)C * blockIdx.z / gridDim.z);
+    cw = (int)((int64_t)C * (blockIdx.z + 1) / gridDim.z) - cb;
+  }
+  const int c0 = cb + (cw * kp) / KP, n = (cw * (kp + 1)) / KP - (cw * kp) / KP;
   // fused: K part kp's rows, block b = i ntok + token (chunk c0 + i), 128 codes + 16 bytes of padding each,
   // quantized by the part's M waves together (wave w % M takes blocks 4 P (w % M) + 0 .. 4 P - 1), then one
   // spare row per wave that takes the stores of lanes past the part's blocks (no branch around the math:
@@ -462,7 +469,7 @@ __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
     bool first = true;
 #pragma unroll
     for (int v = 0; v < KP; ++v) {
-      if ((C * (v + 1)) / KP == (C * v) / KP) continue;
+      if ((cw * (v + 1)) / KP == (cw * v) / KP) continue;
       const float4 r = red[w % M + M * v][ft][lane];
       if (first) {
         o4 = r;
@@ -499,6 +506,10 @@ __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
   const int local = 16 * (ft / TM) + nn;
   if (w >= M * TM * NT || local >= ntok || set_raw >= sets) return;
   const size_t o = (size_t)(tok0 + local) * a.N + 16 * (tile + ft % TM) + 4 * q;
+  if (gridDim.z > 1) {
+    *reinterpret_cast<float4*>(a.partial + (size_t)blockIdx.z * a.T * a.N + o) = o4;
+    return;
+  }
   uint2 packed;
   packed.x = mx::bf16_bits(o4.x) | (mx::bf16_bits(o4.y) << 16);
   packed.y = mx::bf16_bits(o4.z) | (mx::bf16_bits(o4.w) << 16);
@@ -714,17 +725,16 @@ int check_fp8_shape(int N, int K, int block, const char* who) {
 // sums cost a write and a read of splits x T x N floats and a reduce launch), then about 512, every split keeping 8
 // chunks. 2112 x 7168 at T = 2048 (144 workgroups) ran 97 us per call unsplit against 110 us with 4 splits (MI355X,
 // quantizer included).
-int fp8_splits(int N, int K, int T) {
-  if (T <= kGemvMaxTokens) return 1;
+int fp8_gemm_splits(int N, int K, int T) {
   const int base_wgs = ((N / 64 + 3) / 4) * ((T + kGemmTok - 1) / kGemmTok);
   if (base_wgs >= 128) return 1;
   return std::max(1, std::min({8, (K / 128) / 8, (512 + base_wgs - 1) / base_wgs}));
 }
 
-// Shape of the decode GEMV: W waves a workgroup, M tile sets of TM tiles.
+// Shape of the decode GEMV: W waves a workgroup, M tile sets of TM tiles, K split over S workgroups.
 struct RowShape {
-  int W, M, TM;
-  int parts() const { return W / M; }
+  int W, M, TM, S = 1;
+  int parts() const { return W / M; }   // K parts of a workgroup
 };
 
 // Gate/up of the FP8 expert. The 5120 x 2304 expert (two or four launches), us at 1 / 4 / 16 tokens: 13.7 / 17.8 / 20.4
@@ -745,11 +755,30 @@ RowShape fp8_row_shape(int N, int K, int T) {
   //   / 16 tokens, 4 x 1 x 2 22.3 / 22.5 / 22.4 / 23.4; 5120 x 2304: 8 x 2 x 1 5.0 / 7.9 / 8.0 / 8.5, 16 x 2 x 1 6.1 / 6.6 /
   //   8.7 / 9.0, 4 x 1 x 2 5.1 / 7.6 / 7.7 / 8.2.
   const int tiles = N / 16, C = K / 128;
-  if (tiles <= 256) return {T <= 2 && C >= 56 ? 8 : 4, 1, 1};
+  if (tiles <= 256) {
+    RowShape sh{T <= 2 && C >= 56 ? 8 : 4, 1, 1};
+    // Where the tiles leave CUs idle and a part would run through more than 16 chunks, K is split over as many workgroups
+    // as fill the 256 CUs, 32 chunks or more each, and a second launch adds the splits (about 2.5 us). Block 32, us without
+    // / with, at 1 / 8 / 32 tokens: 512 x 12288 - / 10.8 -> 9.4 / 16.1 -> 12.0, 512 x 16384 - / 12.4 -> 9.9 / 19.0 -> 12.1,
+    // 512 x 65536 34.6 -> 12.6 / 34.2 -> 17.2 / 59.4 -> 25.1, 1280 x 32768 21.0 -> 12.2 / 20.8 -> 15.0 / 34.6 -> 22.0. With
+    // 16 chunks a part the second launch costs as much as it saves: 64 x 16384 8.4 -> 7.6 at one token, 512 x 8192 8.5 ->
+    // 8.8 at 8; with tiles for more than half the CUs it loses: 2112 x 16384 10.1 -> 13.0 and 13.7 -> 16.2.
+    if (C > 16 * sh.W) sh.S = std::max(1, std::min({16, 256 / tiles, C / 32}));
+    return sh;
+  }
   if (tiles >= 1024) return T == 3 || T == 4 ? RowShape{8, 2, 2} : RowShape{4, 1, 2};
   if (T <= 2 && C < 64) return {8, 2, 1};
   if (T <= 4) return {16, 2, 1};
   return {4, 1, 2};
+}
+
+// K splits of a call, and the bytes of their partial sums.
+int fp8_splits(int N, int K, int T) {
+  return T <= kGemvMaxTokens ? fp8_row_shape(N, K, T).S : fp8_gemm_splits(N, K, T);
+}
+uint64_t fp8_partial_bytes(int N, int K, int T) {
+  const int splits = fp8_splits(N, K, T);
+  return splits > 1 ? (uint64_t)splits * T * N * sizeof(float) : 0;
 }
 
 // Fused quantization passes (4 blocks of 128 each per wave) for a K part's chunks x the tokens, shared by the
@@ -757,7 +786,7 @@ RowShape fp8_row_shape(int N, int K, int T) {
 // launch).
 int fp8_fused_passes(const RowShape& sh, int K, int T) {
   if (T > kFusedMaxTokens) return 0;
-  const int blocks = ((K / 128 + sh.parts() - 1) / sh.parts()) * T;
+  const int parts = sh.parts() * sh.S, blocks = ((K / 128 + parts - 1) / parts) * T;
   if (blocks > kTileQRows) return 0;
   const int per_wave = (blocks + sh.M - 1) / sh.M;
   return per_wave <= 4 ? 1 : per_wave <= 8 ? 2 : 4;
@@ -765,11 +794,11 @@ int fp8_fused_passes(const RowShape& sh, int K, int T) {
 
 // fp8_row_gemv_kernel of shape (W, M, TM): P fused quantization passes, or P = 0 when x comes quantized.
 template <int kBlock, int W, int M, int TM, bool kPair = false>
-void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st) {
+void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
   const int sets = kPair ? a.N / 16 : a.N / 16 / TM;
   const dim3 threads(64 * W);
   auto go = [&](auto kernel, int tokens = kTok) {
-    hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens), threads, 0, st, a);
+    hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens, S), threads, 0, st, a);
   };
   if constexpr (M == 1 && !kPair)   // the shapes of more than 8 tokens
     if (a.T > kTok) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
@@ -783,8 +812,8 @@ void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st) {
 
 template <int kBlock>
 void launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st) {
-  if (sh.W == 4 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 4, 1, 1>(a, P, st);
-  else if (sh.W == 8 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 8, 1, 1>(a, P, st);
+  if (sh.W == 4 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 4, 1, 1>(a, P, st, sh.S);
+  else if (sh.W == 8 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 8, 1, 1>(a, P, st, sh.S);
   else if (sh.W == 4 && sh.M == 1 && sh.TM == 2) launch_row_gemv<kBlock, 4, 1, 2>(a, P, st);
   else if (sh.W == 8 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 8, 2, 1>(a, P, st);
   else if (sh.W == 8 && sh.M == 2 && sh.TM == 2) launch_row_gemv<kBlock, 8, 2, 2>(a, P, st);
@@ -811,9 +840,9 @@ int launch_quant_ordered(int block, const uint16_t* x, uint8_t* q, void* s, int 
   return MX_OK;
 }
 
-// The product on quantized activations: the row GEMV (T <= 32: no K split across workgroups) or the tiled GEMM,
-// with K split over fp8_splits(N, K, T) workgroups whose FP32 partial sums go to `partial` (fp8_splits * T * N
-// floats) and are added in split order by fp8_splitk_reduce_kernel.
+// The product on quantized activations: the row GEMV (T <= 32) or the tiled GEMM, with K split over fp8_splits(N, K, T)
+// workgroups whose FP32 partial sums go to `partial` (fp8_partial_bytes) and are added in split order by
+// fp8_splitk_reduce_kernel.
 // x_fused: the BF16 input when the GEMV quantizes it itself (fp8_fused_ok), else null (q and sc given); ordered: q
 // and sc as launch_quant_ordered wrote them.
 int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8_t* q, const void* sc, int T,
@@ -833,6 +862,7 @@ int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8
   a.partial = partial;
   a.x = x_fused;
   a.ordered = ordered;
+  const int splits = fp8_splits(N, K, T);
   if (T <= kGemvMaxTokens) {
     const RowShape sh = fp8_row_shape(N, K, T);
     const int P = x_fused ? fp8_fused_passes(sh, K, T) : 0;
@@ -840,16 +870,16 @@ int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8
     else launch_row_gemv<128>(sh, a, P, st);
     MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
   } else {
-    const int splits = fp8_splits(N, K, T);
     const dim3 grid((N / 64 + 3) / 4, (T + kGemmTok - 1) / kGemmTok, splits);
     if (block == 32) hipLaunchKernelGGL(fp8_gemm_kernel<32>, grid, dim3(kGemmThreads), 0, st, a);
     else hipLaunchKernelGGL(fp8_gemm_kernel<128>, grid, dim3(kGemmThreads), 0, st, a);
-    if (splits > 1) {
-      const int64_t count = (int64_t)T * N;
-      hipLaunchKernelGGL(fp8_splitk_reduce_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, st,
-                         (const float*)partial, splits, count, y, trace);
-      MX_LAUNCH_CHECK("fp8_splitk_reduce_kernel");
-    }
+    MX_LAUNCH_CHECK("fp8_gemm_kernel");
+  }
+  if (splits > 1) {
+    const int64_t count = (int64_t)T * N;
+    hipLaunchKernelGGL(fp8_splitk_reduce_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, st,
+                       (const float*)partial, splits, count, y, trace);
+    MX_LAUNCH_CHECK("fp8_splitk_reduce_kernel");
   }
   return MX_OK;
 }
@@ -914,10 +944,8 @@ int mx_fp8_projection(mx_ctx* ctx, const void* tiled, int32_t N, int32_t K, int3
   const bool ordered = !q_out && !s_out && T <= kGemvMaxTokens;
   const uint64_t rows = ordered ? (T + kTok - 1) / kTok * kTok : T;
   const uint64_t q_b = (rows * K + 255) & ~255ull, s_b = (rows * (K / 32) + 255) & ~255ull;   // 4 scale bytes a chunk
-  const int splits = fp8_splits(N, K, T);
-  const uint64_t p_b = splits > 1 ? (uint64_t)splits * T * N * 4 : 0;
   void* base = nullptr;
-  if (int s = scratch(ctx, q_b + s_b + p_b + 256, &base)) return s;
+  if (int s = scratch(ctx, q_b + s_b + fp8_partial_bytes(N, K, T) + 256, &base)) return s;
   uint8_t* q = q_out ? q_out : (uint8_t*)base;
   void* sc = s_out ? s_out : (void*)((uint8_t*)base + q_b);
   MX_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)sc & 3) == 0, "mx_fp8_projection: q 16-byte, s 4-byte aligned");
@@ -950,8 +978,10 @@ int mx_fp8_grouped_projection(mx_ctx* ctx, const void* tiled, int32_t groups, in
   MX_REQUIRE(((uintptr_t)tiled & 255) == 0 && ((uintptr_t)q & 15) == 0 && ((uintptr_t)s & 3) == 0 &&
                  ((uintptr_t)y & 7) == 0 && ((uintptr_t)trace & 15) == 0,
              "mx_fp8_grouped_projection: tiled 256-byte, q 16-byte, s 4-byte, y 8-byte, trace 16-byte alignment");
-  return launch_fp8_product((const uint8_t*)tiled, N, K, 32, q, s, T, y, trace, nullptr, as_stream(stream), nullptr,
-                            false, rows);
+  void* partial = nullptr;
+  if (int st = scratch(ctx, fp8_partial_bytes(N, K, T), &partial)) return st;
+  return launch_fp8_product((const uint8_t*)tiled, N, K, 32, q, s, T, y, trace, (float*)partial, as_stream(stream),
+                            nullptr, false, rows);
 }
 
 int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const void* w2, int32_t H, int32_t I,
@@ -971,7 +1001,7 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
   auto r256 = [](uint64_t b) { return (b + 255) & ~255ull; };
   const uint64_t sizes[5] = {r256((uint64_t)kTok * H), r256((uint64_t)kTok * H / 32), r256((uint64_t)T * I * 2),
                              r256((uint64_t)kTok * I), r256((uint64_t)kTok * I / 32)};
-  uint64_t total = 0;
+  uint64_t total = fp8_partial_bytes(H, I, T);
   for (uint64_t b : sizes) total += b;
   void* base = nullptr;
   if (int s = scratch(ctx, total, &base)) return s;
@@ -981,6 +1011,7 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
     buf[i] = cur;
     cur += sizes[i];
   }
+  float* partial = (float*)cur;   // of the down product
   uint8_t* q = (stages && stages->q) ? stages->q : buf[0];
   uint8_t* s = (stages && stages->s) ? stages->s : buf[1];
   uint16_t* din = (stages && stages->down_input) ? stages->down_input : (uint16_t*)buf[2];
@@ -1021,10 +1052,10 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
   MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
   const bool own_dq = (!stages || (!stages->down_q && !stages->down_s)) && ((uintptr_t)din & 15) == 0;
   if (own_dq && fp8_fused_ok(H, I, T) && !overlap(din, xi, y, xh))
-    return launch_fp8_product((const uint8_t*)w2, H, I, 32, nullptr, nullptr, T, y, nullptr, nullptr, st, din);
+    return launch_fp8_product((const uint8_t*)w2, H, I, 32, nullptr, nullptr, T, y, nullptr, partial, st, din);
   if (int e = own_dq ? launch_quant_ordered(32, din, dq, ds, T, I, st) : mx_act_quant32(ctx, din, dq, ds, T, I, stream))
     return e;
-  return launch_fp8_product((const uint8_t*)w2, H, I, 32, dq, ds, T, y, nullptr, nullptr, st, nullptr, own_dq);
+  return launch_fp8_product((const uint8_t*)w2, H, I, 32, dq, ds, T, y, nullptr, partial, st, nullptr, own_dq);
 }
 
 }  // extern "C"
