@@ -48,9 +48,10 @@ def test_split_alike_with_and_without_codes(gpu_ctx, block, tokens):
     np.testing.assert_array_equal(y_f, y_q)
 
 
-def test_weight_scales_past_64_chunks_of_two_tiles_a_wave(gpu_ctx):
-    """Block 128, two tiles a wave (a ring of 3 chunks): 268 chunks in 4 K parts of 67."""
-    check_exact(gpu_ctx, 128, 4160, 34304, 5)
+@pytest.mark.parametrize("rows,width,tokens", [(4160, 34304, 5), (2112, 33792, 3)])
+def test_weight_scales_past_64_chunks_of_a_part(gpu_ctx, rows, width, tokens):
+    """Block 128, two tiles a wave (a ring of 3 chunks) and one (of 4): 4 K parts of 67 and of 66 chunks."""
+    check_exact(gpu_ctx, 128, rows, width, tokens)
 
 
 def test_split_down_product_of_the_expert():

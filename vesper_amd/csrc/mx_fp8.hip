@@ -742,21 +742,35 @@ struct RowShape {
 // W1, W3, SwiGLU, quantizer, W2). Two launches of about 6 us for 35 MB: their ramps and drains bound it now.
 constexpr RowShape kPairShape{8, 1, 2};
 
+// Whether `parts` K parts of C chunks can quantize T tokens themselves: a part's chunks x tokens fit its LDS rows.
+bool fp8_fits(int parts, int C, int T) { return T <= kFusedMaxTokens && (C + parts - 1) / parts * T <= kTileQRows; }
+
 RowShape fp8_row_shape(int N, int K, int T) {
-  // us per call (quantizer launch included where there is one), weights rotated, W x M x TM:
-  // * up to 256 tiles: one tile a workgroup, 4 K parts, or 8 where one or two tokens leave the waves little else to do
-  //   and the parts stay 7 chunks long. 2112 x 7168: 4 parts 6.6 / 8.8 / 9.9 at 1 / 8 / 16 tokens, 8 parts 5.8 / 9.1 /
-  //   10.1, 16 parts 6.5 / 9.7 / 10.7; 1280 x 5120: 4 parts 5.6 / 7.7 / 8.4, 8 parts 5.8 / 8.7 / 9.5.
-  // * from 1024 tiles: two tiles a wave, 4 K parts; two sets a workgroup where 3 or 4 tokens are quantized in it (the
-  //   two waves of a part share that). 24576 x 1536: 4 x 1 x 2 8.0 / 9.3 / 10.3 / 10.7 at 1 / 4 / 8 / 16 tokens, 8 x 2 x
-  //   2 8.4 / 9.0 / 11.1 / 11.5, one tile a wave (8 x 2 x 1) 8.3 / 9.2 / 11.9 / 12.1.
-  // * between: few tokens, two tiles of 8 K parts (4 where the parts would be short); else two tiles a wave, so that
-  //   each activation operand is loaded for two products. 7168 x 16384: 16 x 2 x 1 20.4 / 22.7 / 22.7 / 24.9 at 1 / 4 / 8
-  //   / 16 tokens, 4 x 1 x 2 22.3 / 22.5 / 22.4 / 23.4; 5120 x 2304: 8 x 2 x 1 5.0 / 7.9 / 8.0 / 8.5, 16 x 2 x 1 6.1 / 6.6 /
-  //   8.7 / 9.0, 4 x 1 x 2 5.1 / 7.6 / 7.7 / 8.2.
+  // us per call (quantizer launch included where there is one), weights rotated, W x M x TM, block 32 unless said.
+  // * up to 4 chunks, more than 256 tiles or 16 tokens: no K parts, four tiles a workgroup. A part without a chunk is
+  //   launched, and waits, for nothing: 12288 x 128 at 4 / 8 / 32 tokens 7.1 / 6.4 / 6.9 with the shapes below, 3.3 / 5.5 /
+  //   6.1 so; 24576 x 512 6.9 / 8.8 / 11.3 and 5.0 / 7.2 / 8.7. Few tiles and tokens are the faster for the parts (512 rows
+  //   block 128, 4 tokens 3.2 / 3.5).
+  // * up to 256 tiles: one tile a workgroup, 4 K parts; 8 where those quantize the call and 4 cannot, or where they
+  //   shorten the chains and the quantization enough. 2112 rows, 4 parts / 8 parts: 1 token of 32 / 40 / 56 / 64 chunks 4.8
+  //   / 4.9, 6.0 / 6.2, 6.9 / 6.7, 7.3 / 7.1 (block 128 4.8 / 5.0, 6.1 / 5.8, 6.8 / 6.0, 7.1 / 6.5), 72 10.2 / 7.7; 2 tokens
+  //   of 20 / 24 / 32 / 40 5.1 / 5.1, 5.2 / 4.9, 5.5 / 5.2, 7.9 / 6.7, of 72 10.4 / 11.2; 3 of 20 5.1 / 5.8, 4 of 16 4.6 /
+  //   4.7, of 20 6.8 / 5.9, of 40 7.9 / 8.8; 16 of 56 9.9 / 10.1.
+  // * between: two tiles of 4 K parts where those quantize the call, else of 8 where those do, else two tiles a wave, so
+  //   that each activation operand is loaded for two products. 7168 rows, 8 x 2 x 1 / 16 x 2 x 1 / 4 x 1 x 2: 1 token of 32
+  //   / 64 / 72 / 128 chunks 7.7 / 8.3 / 7.9, 12.3 / 12.4 / 12.9, 15.8 / 14.1 / 15.1, 23.3 / 21.5 / 23.8; 2 of 32 / 40 / 72
+  //   7.9 / 8.2 / 8.4, 11.5 / 10.3 / 11.3, 15.9 / 17.6 / 15.2; 4 of 16 / 20 / 32 / 40 5.4 / 6.4 / 6.1, 8.7 / 7.2 / 8.1, 10.1
+  //   / 8.5 / 10.4, 11.5 / 13.2 / 11.3.
+  // * from 1024 tiles: two tiles a wave, 4 K parts, but for 3 or 4 tokens that 4 parts quantize two sets a workgroup (the
+  //   two waves of a part share that), of two tiles up to 12 chunks (a part's chunks are its ring) and of one above, and
+  //   for up to 4 tokens quantized before from 32 chunks two sets of one tile. 24576 rows, 4 x 1 x 2 / 8 x 2 x 2 / 8 x 2 x
+  //   1 at 4 tokens of 10 / 12 / 16 chunks 9.3 / 8.8 / 8.9, 9.9 / 9.3 / 9.5, 12.7 / 13.2 / 11.1, and, quantized before, of
+  //   18 / 24 / 32 / 40 14.6 / 15.5 / 15.3, 16.7 / 17.5 / 18.2, 21.6 / 21.9 / 20.7, 25.1 / 26.8 / 24.9 (block 128 of 32 20.7
+  //   / 22.1 / 19.7; 16384 x 8192 at 2 tokens 26.4 with the first, 24.4 with the last).
   const int tiles = N / 16, C = K / 128;
+  if (C <= 4 && (tiles > 256 || T > kTok)) return {4, 4, 1};
   if (tiles <= 256) {
-    RowShape sh{T <= 2 && C >= 56 ? 8 : 4, 1, 1};
+    RowShape sh{fp8_fits(8, C, T) && (!fp8_fits(4, C, T) || (T <= 2 && C * T >= 48)) ? 8 : 4, 1, 1};
     // Where the tiles leave CUs idle and a part would run through more than 16 chunks, K is split over as many workgroups
     // as fill the 256 CUs, 32 chunks or more each, and a second launch adds the splits (about 2.5 us). Block 32, us without
     // / with, at 1 / 8 / 32 tokens: 512 x 12288 - / 10.8 -> 9.4 / 16.1 -> 12.0, 512 x 16384 - / 12.4 -> 9.9 / 19.0 -> 12.1,
@@ -766,9 +780,13 @@ RowShape fp8_row_shape(int N, int K, int T) {
     if (C > 16 * sh.W) sh.S = std::max(1, std::min({16, 256 / tiles, C / 32}));
     return sh;
   }
-  if (tiles >= 1024) return T == 3 || T == 4 ? RowShape{8, 2, 2} : RowShape{4, 1, 2};
-  if (T <= 2 && C < 64) return {8, 2, 1};
-  if (T <= 4) return {16, 2, 1};
+  if (tiles >= 1024) {
+    if (!fp8_fits(4, C, T)) return T <= kFusedMaxTokens && C >= 32 ? RowShape{8, 2, 1} : RowShape{4, 1, 2};
+    if (T < 3) return {4, 1, 2};
+    return {8, 2, C <= 12 ? 2 : 1};
+  }
+  if (fp8_fits(4, C, T)) return {8, 2, 1};
+  if (fp8_fits(8, C, T)) return {16, 2, 1};
   return {4, 1, 2};
 }
 
@@ -800,7 +818,7 @@ void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
   auto go = [&](auto kernel, int tokens = kTok) {
     hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens, S), threads, 0, st, a);
   };
-  if constexpr (M == 1 && !kPair)   // the shapes of more than 8 tokens
+  if constexpr (M == 1 && !kPair)
     if (a.T > kTok) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
   if (P == 0) go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair>);
   if (P == 1) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair>);
@@ -814,6 +832,7 @@ template <int kBlock>
 void launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st) {
   if (sh.W == 4 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 4, 1, 1>(a, P, st, sh.S);
   else if (sh.W == 8 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 8, 1, 1>(a, P, st, sh.S);
+  else if (sh.W == 4 && sh.M == 4 && sh.TM == 1) launch_row_gemv<kBlock, 4, 4, 1>(a, P, st);
   else if (sh.W == 4 && sh.M == 1 && sh.TM == 2) launch_row_gemv<kBlock, 4, 1, 2>(a, P, st);
   else if (sh.W == 8 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 8, 2, 1>(a, P, st);
   else if (sh.W == 8 && sh.M == 2 && sh.TM == 2) launch_row_gemv<kBlock, 8, 2, 2>(a, P, st);
