@@ -818,8 +818,12 @@ void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
   auto go = [&](auto kernel, int tokens = kTok) {
     hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens, S), threads, 0, st, a);
   };
+  // More than 16 tokens: both token tiles in a workgroup, so that the weights are read once -- but in two workgroups
+  // where the codes come as rows (16 pieces of 64 bytes an operand) and two workgroups a tile still fit the CUs: the
+  // grouped product of 8 x 64 / 8 x 256 rows of 4096 at 32 tokens 9.0 / 9.2 us in one, 6.3 / 6.5 in two (8 x 512 9.9 and
+  // 11.1, 8 x 1024 12.8 and 14.7).
   if constexpr (M == 1 && !kPair)
-    if (a.T > kTok) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
+    if (a.T > kTok && (a.ordered || a.N > 2048)) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
   if (P == 0) go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair>);
   if (P == 1) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair>);
   if constexpr (8 * M <= kTileQRows)
