@@ -168,11 +168,13 @@ __device__ __forceinline__ uint2 quantize8(const uint4& raw, uint32_t& scale) {
 // operand of 16 tokens is two linear 1 KB loads instead of 32 row pieces of 64 bytes, and its scales 64 contiguous
 // bytes instead of 16 rows. Token tile tt (16 tokens), chunk c: half h of lane (q, n) -- token 16 tt + n, K 64 h + 16 q
 // + 0..15 of the chunk -- at (tt C + c) 2048 + 1024 h + 16 (16 q + n); the scales (block 32: four E8M0 codes, block 128:
-// FP32) at (tt C + c) 64 + 4 n. 16 lanes per (token, chunk).
+// FP32) at (tt C + c) 64 + 4 n. 16 lanes per (token, chunk). q_rows, s_rows (nullable): the codes and scales as rows, too,
+// for a caller that asks for them -- the same bytes as the quantizer launches write.
 template <int kBlock>
 __global__ __launch_bounds__(256) void fp8_quant_ordered_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ q,
-                                                                uint8_t* __restrict__ s, int T, int C) {
-  const int b = (blockIdx.x * 256 + threadIdx.x) >> 4, sub = threadIdx.x & 15;
+                                                                uint8_t* __restrict__ s, uint8_t* __restrict__ q_rows,
+                                                                uint8_t* __restrict__ s_rows, int T, int C) {
+  const int b = (int)(blockIdx.x * 16 + (threadIdx.x >> 4)), sub = threadIdx.x & 15;
   if (b >= T * C) return;   // whole groups of 16 lanes
   const int t = b / C, c = b - t * C, n = t & 15;
   uint32_t scale;
@@ -182,10 +184,17 @@ __global__ __launch_bounds__(256) void fp8_quant_ordered_kernel(const uint16_t* 
   // values 8 sub .. 8 sub + 7: half sub / 8, lane group (sub / 2) % 4, upper or lower 8 bytes by sub % 2
   *reinterpret_cast<uint2*>(q + at * 2048 + 1024 * (sub >> 3) + 16 * (16 * ((sub >> 1) & 3) + n) + 8 * (sub & 1)) = codes;
   if constexpr (kBlock == 32) {
-    if ((sub & 3) == 0) s[at * 64 + 4 * n + (sub >> 2)] = (uint8_t)scale;
+    if ((sub & 3) == 0) {
+      s[at * 64 + 4 * n + (sub >> 2)] = (uint8_t)scale;
+      if (s_rows) s_rows[(size_t)b * 4 + (sub >> 2)] = (uint8_t)scale;
+    }
   } else {
-    if (sub == 0) *reinterpret_cast<uint32_t*>(s + at * 64 + 4 * n) = scale;
+    if (sub == 0) {
+      *reinterpret_cast<uint32_t*>(s + at * 64 + 4 * n) = scale;
+      if (s_rows) *reinterpret_cast<uint32_t*>(s_rows + (size_t)b * 4) = scale;
+    }
   }
+  if (q_rows) *reinterpret_cast<uint2*>(q_rows + (size_t)b * 128 + 8 * sub) = codes;
 }
 
 struct Fp8Args {
@@ -854,11 +863,12 @@ bool overlap(const void* a, uint64_t na, const void* b, uint64_t nb) {
 bool fp8_fused_ok(int N, int K, int T) { return T <= kFusedMaxTokens && fp8_fused_passes(fp8_row_shape(N, K, T), K, T) > 0; }
 
 // fp8_quant_ordered_kernel: T tokens' codes and scales into buffers of T rounded up to 16 rows.
-int launch_quant_ordered(int block, const uint16_t* x, uint8_t* q, void* s, int T, int K, hipStream_t st) {
+int launch_quant_ordered(int block, const uint16_t* x, uint8_t* q, void* s, int T, int K, hipStream_t st,
+                         uint8_t* q_rows = nullptr, void* s_rows = nullptr) {
   const int C = K / 128;
   const dim3 grid((unsigned)(((int64_t)T * C + 15) / 16));
-  if (block == 32) hipLaunchKernelGGL(fp8_quant_ordered_kernel<32>, grid, dim3(256), 0, st, x, q, (uint8_t*)s, T, C);
-  else hipLaunchKernelGGL(fp8_quant_ordered_kernel<128>, grid, dim3(256), 0, st, x, q, (uint8_t*)s, T, C);
+  hipLaunchKernelGGL(block == 32 ? fp8_quant_ordered_kernel<32> : fp8_quant_ordered_kernel<128>, grid, dim3(256), 0, st, x,
+                     q, (uint8_t*)s, q_rows, (uint8_t*)s_rows, T, C);
   MX_LAUNCH_CHECK("fp8_quant_ordered_kernel");
   return MX_OK;
 }
@@ -963,22 +973,26 @@ int mx_fp8_projection(mx_ctx* ctx, const void* tiled, int32_t N, int32_t K, int3
                  ((uintptr_t)trace & 15) == 0,
              "mx_fp8_projection: tiled 256-byte, x 16-byte, y 8-byte and trace 16-byte alignment required");
   hipStream_t st = as_stream(stream);
-  // the decode GEMV's own codes come in its load order, in whole tiles of 16 tokens
-  const bool ordered = !q_out && !s_out && T <= kGemvMaxTokens;
+  MX_REQUIRE(((uintptr_t)q_out & 15) == 0 && ((uintptr_t)s_out & 3) == 0,
+             "mx_fp8_projection: q 16-byte, s 4-byte aligned");
+  // The decode GEMV's codes come in its load order, in whole tiles of 16 tokens, and the rows that a caller asks for are
+  // written beside them; up to 4 tokens' rows are read as they are (us, rows / load order: 2112 x 7168 block 128 at one
+  // token 8.7 / 9.1, block 32 at 16 12.4 / 10.6, 512 x 7168 at 32 17.8 / 11.9, 7168 x 16384 at 32 43.3 / 29.5).
+  const bool codes = q_out || s_out;
+  const bool ordered = T <= kGemvMaxTokens && (!codes || T > kFusedMaxTokens);
   const uint64_t rows = ordered ? (T + kTok - 1) / kTok * kTok : T;
   const uint64_t q_b = (rows * K + 255) & ~255ull, s_b = (rows * (K / 32) + 255) & ~255ull;   // 4 scale bytes a chunk
   void* base = nullptr;
   if (int s = scratch(ctx, q_b + s_b + fp8_partial_bytes(N, K, T) + 256, &base)) return s;
-  uint8_t* q = q_out ? q_out : (uint8_t*)base;
-  void* sc = s_out ? s_out : (void*)((uint8_t*)base + q_b);
-  MX_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)sc & 3) == 0, "mx_fp8_projection: q 16-byte, s 4-byte aligned");
+  uint8_t* q = q_out && !ordered ? q_out : (uint8_t*)base;
+  void* sc = s_out && !ordered ? s_out : (void*)((uint8_t*)base + q_b);
   float* partial = (float*)((uint8_t*)base + q_b + s_b);
   const uint64_t x_b = (uint64_t)T * K * 2, y_b = (uint64_t)T * N * 2;
-  if (!q_out && !s_out && fp8_fused_ok(N, K, T) && !overlap(x, x_b, y, y_b) &&
+  if (!codes && fp8_fused_ok(N, K, T) && !overlap(x, x_b, y, y_b) &&
       !overlap(x, x_b, trace, 2 * y_b))   // the GEMV quantizes x itself
     return launch_fp8_product((const uint8_t*)tiled, N, K, block, nullptr, nullptr, T, y, trace, partial, st, x);
   if (ordered) {
-    if (int s = launch_quant_ordered(block, x, q, sc, T, K, st)) return s;
+    if (int s = launch_quant_ordered(block, x, q, sc, T, K, st, q_out, s_out)) return s;
   } else if (block == 32) {
     if (int s = mx_act_quant32(ctx, x, q, (uint8_t*)sc, T, K, stream)) return s;
   } else {
