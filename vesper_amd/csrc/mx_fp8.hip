@@ -30,6 +30,7 @@ using mxd::ldg32;
 using mxd::ldgf;
 using mxd::mfma_fp8_fp8;
 using mxd::v4f;
+using mxi::fail;
 
 constexpr int kTiles = 4;   // 16-row MFMA tiles per workgroup: 64 weight rows
 constexpr int kTok = 16;    // token columns per MFMA
@@ -746,7 +747,7 @@ struct RowShape {
   int parts() const { return W / M; }   // K parts of a workgroup
 };
 
-// Gate/up of the FP8 expert. The 5120 x 2304 expert (two or four launches), us at 1 / 4 / 16 tokens: 13.7 / 17.8 / 20.4
+// Gate/up of the FP8 expert. The 5120 x 2304 expert (two / three / four launches), us at 1 / 4 / 16 tokens: 13.7 / 17.8 / 20.4
 // with 8 waves, 14.7 / 17.8 / 21.2 with 16, 14.1 / 18.2 / 20.0 with 4; 31.6 / 33.0 / 34.7 as six launches (quantizer,
 // W1, W3, SwiGLU, quantizer, W2). Two launches of about 6 us for 35 MB: their ramps and drains bound it now.
 constexpr RowShape kPairShape{8, 1, 2};
@@ -782,8 +783,8 @@ RowShape fp8_row_shape(int N, int K, int T) {
     RowShape sh{fp8_fits(8, C, T) && (!fp8_fits(4, C, T) || (T <= 2 && C * T >= 48)) ? 8 : 4, 1, 1};
     // Where the tiles leave CUs idle and a part would run through more than 16 chunks, K is split over as many workgroups
     // as fill the 256 CUs, 32 chunks or more each, and a second launch adds the splits (about 2.5 us). Block 32, us without
-    // / with, at 1 / 8 / 32 tokens: 512 x 12288 - / 10.8 -> 9.4 / 16.1 -> 12.0, 512 x 16384 - / 12.4 -> 9.9 / 19.0 -> 12.1,
-    // 512 x 65536 34.6 -> 12.6 / 34.2 -> 17.2 / 59.4 -> 25.1, 1280 x 32768 21.0 -> 12.2 / 20.8 -> 15.0 / 34.6 -> 22.0. With
+    // / with, at 1 / 8 / 32 tokens: 512 x 12288 - / 10.8 -> 9.5 / 16.1 -> 11.9, 512 x 16384 - / 12.4 -> 9.7 / 19.0 -> 12.2,
+    // 512 x 65536 34.6 -> 12.0 / 34.2 -> 15.6 / 59.4 -> 21.5, 1280 x 32768 21.0 -> 14.6 / 20.8 -> 15.1 / 34.6 -> 22.1. With
     // 16 chunks a part the second launch costs as much as it saves: 64 x 16384 8.4 -> 7.6 at one token, 512 x 8192 8.5 ->
     // 8.8 at 8; with tiles for more than half the CUs it loses: 2112 x 16384 10.1 -> 13.0 and 13.7 -> 16.2.
     if (C > 16 * sh.W) sh.S = std::max(1, std::min({16, 256 / tiles, C / 32}));
@@ -819,37 +820,47 @@ int fp8_fused_passes(const RowShape& sh, int K, int T) {
   return per_wave <= 4 ? 1 : per_wave <= 8 ? 2 : 4;
 }
 
-// fp8_row_gemv_kernel of shape (W, M, TM): P fused quantization passes, or P = 0 when x comes quantized.
+// fp8_row_gemv_kernel of shape (W, M, TM): P fused quantization passes, or P = 0 when x comes quantized. A combination
+// that fp8_row_shape does not make has no kernel and is an error, not a call that leaves y as it was.
 template <int kBlock, int W, int M, int TM, bool kPair = false>
-void launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
+int launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
   const int sets = kPair ? a.N / 16 : a.N / 16 / TM;
-  const dim3 threads(64 * W);
   auto go = [&](auto kernel, int tokens = kTok) {
-    hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens, S), threads, 0, st, a);
+    hipLaunchKernelGGL(kernel, dim3((sets + M - 1) / M, (a.T + tokens - 1) / tokens, S), dim3(64 * W), 0, st, a);
+    MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
+    return MX_OK;
   };
   // More than 16 tokens: both token tiles in a workgroup, so that the weights are read once -- but in two workgroups
   // where the codes come as rows (16 pieces of 64 bytes an operand) and two workgroups a tile still fit the CUs: the
   // grouped product of 8 x 64 / 8 x 256 rows of 4096 at 32 tokens 9.0 / 9.2 us in one, 6.3 / 6.5 in two (8 x 512 9.9 and
   // 11.1, 8 x 1024 12.8 and 14.7).
-  if constexpr (M == 1 && !kPair)
-    if (a.T > kTok && (a.ordered || a.N > 2048)) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
-  if (P == 0) go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair>);
-  if (P == 1) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair>);
+  if constexpr (W == 4 && M == 1)
+    if (P == 0 && a.T > kTok && (a.ordered || a.N > 2048))
+      return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
+  if (P == 0) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair>);
+  if constexpr (W / M < 8 || kPair)   // 8 parts are only chosen for more blocks than one pass takes
+    if (P == 1) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair>);
   if constexpr (8 * M <= kTileQRows)
-    if (P == 2) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 2, kPair>);
+    if (P == 2) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 2, kPair>);
   if constexpr (16 * M <= kTileQRows)
-    if (P == 4) go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 4, kPair>);
+    if (P == 4) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 4, kPair>);
+  return fail(MX_ERR_STATE, "FP8 GEMV: %d passes of the %d x %d x %d shape have no kernel", P, W, M, TM);
 }
 
 template <int kBlock>
-void launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st) {
-  if (sh.W == 4 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 4, 1, 1>(a, P, st, sh.S);
-  else if (sh.W == 8 && sh.M == 1 && sh.TM == 1) launch_row_gemv<kBlock, 8, 1, 1>(a, P, st, sh.S);
-  else if (sh.W == 4 && sh.M == 4 && sh.TM == 1) launch_row_gemv<kBlock, 4, 4, 1>(a, P, st);
-  else if (sh.W == 4 && sh.M == 1 && sh.TM == 2) launch_row_gemv<kBlock, 4, 1, 2>(a, P, st);
-  else if (sh.W == 8 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 8, 2, 1>(a, P, st);
-  else if (sh.W == 8 && sh.M == 2 && sh.TM == 2) launch_row_gemv<kBlock, 8, 2, 2>(a, P, st);
-  else if (sh.W == 16 && sh.M == 2 && sh.TM == 1) launch_row_gemv<kBlock, 16, 2, 1>(a, P, st);
+int launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st) {
+  const int shape = 100 * sh.W + 10 * sh.M + sh.TM;
+  if (sh.S > 1 && shape != 411) return fail(MX_ERR_STATE, "FP8 GEMV: shape %d does not split K", shape);
+  switch (shape) {
+    case 411: return launch_row_gemv<kBlock, 4, 1, 1>(a, P, st, sh.S);
+    case 811: return launch_row_gemv<kBlock, 8, 1, 1>(a, P, st);
+    case 412: return launch_row_gemv<kBlock, 4, 1, 2>(a, P, st);
+    case 441: return launch_row_gemv<kBlock, 4, 4, 1>(a, P, st);
+    case 821: return launch_row_gemv<kBlock, 8, 2, 1>(a, P, st);
+    case 822: return launch_row_gemv<kBlock, 8, 2, 2>(a, P, st);
+    case 1621: return launch_row_gemv<kBlock, 16, 2, 1>(a, P, st);
+  }
+  return fail(MX_ERR_STATE, "FP8 GEMV: shape %d has no kernel", shape);
 }
 
 // Whether a[0 .. na) and b[0 .. nb) share bytes (a null pointer shares none). A launch that quantizes its own input
@@ -899,9 +910,7 @@ int launch_fp8_product(const uint8_t* blob, int N, int K, int block, const uint8
   if (T <= kGemvMaxTokens) {
     const RowShape sh = fp8_row_shape(N, K, T);
     const int P = x_fused ? fp8_fused_passes(sh, K, T) : 0;
-    if (block == 32) launch_row_gemv<32>(sh, a, P, st);
-    else launch_row_gemv<128>(sh, a, P, st);
-    MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
+    if (int s = block == 32 ? launch_row_gemv<32>(sh, a, P, st) : launch_row_gemv<128>(sh, a, P, st)) return s;
   } else {
     const dim3 grid((N / 64 + 3) / 4, (T + kGemmTok - 1) / kGemmTok, splits);
     if (block == 32) hipLaunchKernelGGL(fp8_gemm_kernel<32>, grid, dim3(kGemmThreads), 0, st, a);
@@ -1085,8 +1094,7 @@ int mx_fp8_expert_forward(mx_ctx* ctx, const void* w1, const void* w3, const voi
   if (p1) a.x = x;
   else if (int e = own_q ? launch_quant_ordered(32, x, q, s, T, H, st) : mx_act_quant32(ctx, x, q, s, T, H, stream))
     return e;
-  launch_row_gemv<32, kPairShape.W, 1, 2, true>(a, p1, st);
-  MX_LAUNCH_CHECK("fp8_row_gemv_kernel");
+  if (int e = launch_row_gemv<32, kPairShape.W, 1, 2, true>(a, p1, st)) return e;
   const bool own_dq = (!stages || (!stages->down_q && !stages->down_s)) && ((uintptr_t)din & 15) == 0;
   if (own_dq && fp8_fused_ok(H, I, T) && !overlap(din, xi, y, xh))
     return launch_fp8_product((const uint8_t*)w2, H, I, 32, nullptr, nullptr, T, y, nullptr, partial, st, din);
