@@ -896,7 +896,6 @@ struct SharedCopies {
   uint32_t lds;           // the ring's LDS byte address
   int stage_bytes;
   bool copies_scale;
-  __device__ __forceinline__ int copies() const { return n_act + (copies_scale ? 1 : 0); }
   __device__ __forceinline__ void issue(int g, int st) const {
     const uint32_t base = lds + st * stage_bytes;
     const int left = n - kStageChunks * g;   // the row's chunks from this stage on
@@ -988,12 +987,11 @@ __device__ __forceinline__ float exact_chunk_few(const uint32_t (&wv)[4], uint32
 
 // The whole K range (n chunks) of tile `wave` of a row group, stage by stage. At the start of stage g a wave waits
 // until its weights and its own copies of stage g have landed, a barrier makes every wave's copies visible, and the
-// wave issues its copies of stage g + kX - 1 (into the ring slot of stage g - 1, which every wave finished reading
-// before this barrier) and, once the stage's weights have left their ring slots, its weights of stage g + kWS; then
-// it multiplies the stage's chunks. Past the end weights load from the dummy page and copies read it, so every stage
-// issues the same loads per wave. When a wave waits at stage g, what it issued after the weights of stage g (stages
-// g - kWS + 1 .. g - 1: copies + kStageChunks loads each) and after its copies of stage g (the weights of stage
-// g - kX + 1 and all of the later stages) may still be in flight.
+// wave issues its copies of stage g + 1 (into the ring slot of stage g - 1, which every wave finished reading before this
+// barrier) and, once the stage's weights have left their ring slots, its weights of stage g + kWStages; then it multiplies
+// the stage's chunks. Past the end weights load from the dummy page and copies read it, so every stage issues the same
+// loads per wave: copies of stage g, then the kStageChunks weights of stage g + 1, are the last before the wait at stage
+// g, so all but kStageChunks loads have landed there, however many copies a wave issues.
 constexpr int kWStages = 2;   // stages of weights in the register ring
 
 template <int kAfter>
@@ -1002,55 +1000,35 @@ __device__ __forceinline__ void vm_wait() {
   __builtin_amdgcn_s_waitcnt(mxd::vm_wait_imm(kAfter));
 }
 
-// wait for this wave's weights and copies of a stage, with `copies` copy instructions per stage (0 .. 5)
-template <int kX, int kCopies>
-__device__ __forceinline__ void wait_stage() {
-  constexpr int kPer = kCopies + kStageChunks;
-  constexpr int kAfterW = (kWStages - 1) * kPer, kAfterC = kStageChunks + (kX - 2) * kPer;
-  vm_wait<(kAfterW < kAfterC ? kAfterW : kAfterC)>();
-}
-
-template <bool kFew, int kX>
+template <bool kFew>
 __device__ __forceinline__ void stream_exact(const uint8_t* wbase, uint32_t woff, const SharedCopies& sc,
                                              uint32_t xaddr, uint32_t caddr, int n, v4f& acc) {
   constexpr int kC = kStageChunks, kWS = kWStages, kW = kWS * kC;
-  const int sb = sc.stage_bytes, n_stages = (n + kC - 1) / kC, copies = sc.copies();
+  static_assert(kXStages == 2 && kWS == 2, "copies of stage g and weights of stage g + 1 are issued together");
+  const int sb = sc.stage_bytes, n_stages = (n + kC - 1) / kC;
   acc = v4f{0.f, 0.f, 0.f, 0.f};
   u32x4_t wr[kW];
   // past the last chunk the base is the dummy page (woff is 16 x lane), selected without a branch
   auto load_w = [&](u32x4_t& r, int c) { r = asm_ldg128_nt(c < n ? wbase + (size_t)c * 4096 : sc.dummy, woff); };
-  // the loads of the stages before 0 in the steady state's order: stage g issues C(g + kX - 1), then W(g + kWS)
-  // (those whose stage index is negative do not exist)
-  constexpr int kPro = kWS > kX - 1 ? kWS : kX - 1;
+  // the loads of the stages before 0 in the steady state's order: W(0), C(0), W(1)
 #pragma unroll
-  for (int vg = -kPro; vg < 0; ++vg) {
-    if (vg + kX - 1 >= 0) sc.issue(vg + kX - 1, vg + kX - 1);
-    if (vg + kWS >= 0) {
+  for (int u = 0; u < kC; ++u) load_w(wr[u], u);
+  sc.issue(0, 0);
 #pragma unroll
-      for (int u = 0; u < kC; ++u) load_w(wr[kC * (vg + kWS) + u], kC * (vg + kWS) + u);
-    }
-  }
-  int slot = 0;   // g % kX
+  for (int u = 0; u < kC; ++u) load_w(wr[kC + u], kC + u);
   for (int g0 = 0; g0 < n_stages; g0 += kWS) {
 #pragma unroll
     for (int gs = 0; gs < kWS; ++gs) {
       const int g = g0 + gs;
       // the waits and ties run for every slot, past the end too: a slot's registers are only released (and
       // reusable by the compiler) once the load that writes them has landed
-      switch (copies) {
-        case 0: wait_stage<kX, 0>(); break;
-        case 1: wait_stage<kX, 1>(); break;
-        case 2: wait_stage<kX, 2>(); break;
-        case 3: wait_stage<kX, 3>(); break;
-        case 4: wait_stage<kX, 4>(); break;
-        default: wait_stage<kX, 5>(); break;
-      }
+      vm_wait<kC>();
 #pragma unroll
       for (int u = 0; u < kC; ++u) asm volatile("" : "+v"(wr[kC * gs + u]));   // landed with the wait above
       // every wave's copies of stage g have landed, and every wave has finished reading stage g - 1, whose slot
       // this stage's copies overwrite (past the last stage only that one is still read)
       if (g <= n_stages) mxd::copy_barrier();
-      sc.issue(g + kX - 1, slot == 0 ? kX - 1 : slot - 1);
+      sc.issue(g + 1, 1 - gs);   // stage g's ring slot is gs
       // the stage's weights leave the ring transposed, and its slots take their next loads at once: no register
       // with a load in flight is touched again, nor merged from two paths, before the wait that ties it
       uint32_t wv[kC][4];
@@ -1062,8 +1040,7 @@ __device__ __forceinline__ void stream_exact(const uint8_t* wbase, uint32_t woff
       }
 #pragma unroll
       for (int u = 0; u < kC; ++u) load_w(wr[kC * gs + u], kC * g + u + kW);
-      const uint32_t xs = xaddr + slot * sb, cs = caddr + slot * sb;
-      slot = slot == kX - 1 ? 0 : slot + 1;
+      const uint32_t xs = xaddr + gs * sb, cs = caddr + gs * sb;
       if (kC * g + kC <= n) {   // a whole stage: no branches between its chunks
 #pragma unroll
         for (int u = 0; u < kC; ++u) {
@@ -1464,8 +1441,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
   const uint32_t caddr = ring0 + kXStageScale + 4 * m + wave;
   const uint8_t* wbase = blob + (size_t)g * chunks * 4096 + (size_t)wave * 1024;
   v4f acc;
-  if (few) stream_exact<true, kXStages>(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
-  else stream_exact<false, kXStages>(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
+  if (few) stream_exact<true>(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
+  else stream_exact<false>(wbase, 16 * lane, sc, xaddr, caddr, (int)chunks, acc);
   // tile `wave` holds the group's W1 rows 8 wave + 0..7 as rows 0-7 and the same W3 rows as rows 8-15: lane (n, q)
   // has token n's sums of tile rows 4q + i, or with few tokens token q's sum of tile row n
   __shared__ __attribute__((aligned(16))) float s_gu[2][kMaxTokens][36];
