@@ -10,6 +10,7 @@ from oracle.expert import expert_reference_stages
 from oracle.formats import bf16_bits
 from oracle.inputs import activations, mxfp4_expert
 from tests.helpers import assert_close
+from tests.test_gpu_bf16_expert import normwise
 from vesper_amd.expert import BF16ActivationExpert
 
 pytestmark = pytest.mark.gpu
@@ -21,10 +22,14 @@ def test_few_tokens(hidden, intermediate):
     arrays = mxfp4_expert(rng, hidden, intermediate, scale_lo=118, scale_hi=120)
     x = activations(rng, 5, hidden)
     with BF16ActivationExpert(arrays, hidden=hidden, intermediate=intermediate) as expert:
-        whole = expert.forward(x)["y"]
-        assert_close(whole, bf16_bits(expert_reference_stages(x, arrays)["y"].astype(np.float32)), "y")
+        whole, ref = expert.forward(x), expert_reference_stages(x, arrays)
+        assert_close(whole["y"], bf16_bits(ref["y"].astype(np.float32)), "y")
+        assert normwise(whole["h"], ref["h"]) < 1e-5
         for t in (1, 2, 3, 4):
-            np.testing.assert_array_equal(expert.forward(x[:t])["y"], whole[:t])
+            got = expert.forward(x[:t])
+            assert normwise(got["h"], ref["h"][:t]) < 1e-5
+            for name in ("h", "y"):
+                np.testing.assert_array_equal(got[name], whole[name][:t], err_msg=name)
 
 
 def test_an_overflowing_token_stays_alone():

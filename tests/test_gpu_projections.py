@@ -176,8 +176,8 @@ def test_exact_through_the_split_k_gemv(block, tokens):
 
 def project_both_ways(proj, ctx, name, bits, rows, width):
     """One projection of BF16 `bits` with the activation codes and scales requested (the quantizer kernel
-    runs first) and without them (block 128 at <= 4 tokens: the GEMV quantizes in LDS). Returns
-    (trace, y) of each."""
+    runs first) and without them (up to 4 tokens that its K parts have room for: the GEMV quantizes in LDS; up
+    to 32: the quantizer writes the GEMV's load order alone). Returns (trace, y) of each."""
     tokens = bits.shape[0]
     x = ctx.upload(bits)
     q = ctx.empty((tokens, width), np.uint8)

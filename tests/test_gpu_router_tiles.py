@@ -1,5 +1,5 @@
-"""The many-token router (8 x 8 tiles, from 25 tokens) gives the bits of the few-token one on every (expert, token): the
-same rows in calls of up to 16 tokens. Expert and token counts that leave partial tiles, one expert, widths below one
+"""The many-token router (8 x 8 tiles, from 25 tokens up to 5120 wide, and wider from 8192 sums) gives the bits of the
+few-token one on every (expert, token): the same rows in calls of up to 16 tokens. Expert and token counts that leave partial tiles, one expert, widths below one
 thread pass, just past one and with a short last pass, and the scores and selection values of a biased router."""
 
 import ctypes as C

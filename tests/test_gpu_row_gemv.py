@@ -52,8 +52,8 @@ def test_shapes_exact_and_alike_with_and_without_codes(gpu_ctx, block, rows, wid
         np.testing.assert_array_equal(y_f, y_q)
 
 
-def test_weight_scales_past_64_chunks_of_a_k_part(gpu_ctx):
-    """Block 128: a wave keeps 64 weight scales in its lanes at a time; 128 x 128 x 8 wide is 128 chunks a part."""
+def test_very_wide_projection(gpu_ctx):
+    """Block 128, 1024 chunks of 64 rows: K shared between 16 workgroups of 4 parts (16 chunks each)."""
     w, sw, x = exact_case(128, 3, 64, 131072, 1, 1, 5)
     x[:, 1::128] = 0.0
     with projections(w, sw, 128) as proj:
