@@ -10,7 +10,7 @@ from tests.test_gpu_row_gemv_split import check_exact
 pytestmark = pytest.mark.gpu
 
 SHORT = [(rows, 128 * chunks, tokens) for rows in (64, 4160, 16448) for chunks in (1, 3, 4, 5) for tokens in (1, 4, 5, 32)]
-FEW = [(192, 128 * chunks, tokens) for tokens, chunks in ((1, 47), (1, 48), (1, 128), (1, 129), (2, 23), (2, 24), (2, 33), (2, 64),
+FEW = [(192, 128 * chunks, tokens) for tokens, chunks in ((1, 55), (1, 56), (1, 128), (1, 129), (2, 27), (2, 28), (2, 33), (2, 64),
                                                          (2, 65), (3, 20), (3, 21), (3, 40), (3, 41), (4, 16), (4, 17),
                                                          (4, 32), (4, 33))]
 BETWEEN = [(4160, 128 * chunks, tokens) for tokens, chunks in ((1, 64), (1, 65), (2, 33), (3, 20), (3, 21), (3, 41), (4, 16),

@@ -169,9 +169,9 @@ __device__ __forceinline__ uint2 quantize8(const uint4& raw, uint32_t& scale) {
 // operand of 16 tokens is two linear 1 KB loads instead of 32 row pieces of 64 bytes, and its scales 64 contiguous
 // bytes instead of 16 rows. Token tile tt (16 tokens), chunk c: half h of lane (q, n) -- token 16 tt + n, K 64 h + 16 q
 // + 0..15 of the chunk -- at (tt C + c) 2048 + 1024 h + 16 (16 q + n); the scales (block 32: four E8M0 codes, block 128:
-// FP32) at (tt C + c) 64 + 4 n. 16 lanes per (token, chunk). q_rows, s_rows (nullable): the codes and scales as rows, too,
-// for a caller that asks for them -- the same bytes as the quantizer launches write.
-template <int kBlock>
+// FP32) at (tt C + c) 64 + 4 n. 16 lanes per (token, chunk). kRows: q_rows, s_rows (either nullable) get the codes and
+// scales as rows, too, for a caller that asks for them -- the same bytes as the quantizer launches write.
+template <int kBlock, bool kRows>
 __global__ __launch_bounds__(256) void fp8_quant_ordered_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ q,
                                                                 uint8_t* __restrict__ s, uint8_t* __restrict__ q_rows,
                                                                 uint8_t* __restrict__ s_rows, int T, int C) {
@@ -187,15 +187,15 @@ __global__ __launch_bounds__(256) void fp8_quant_ordered_kernel(const uint16_t* 
   if constexpr (kBlock == 32) {
     if ((sub & 3) == 0) {
       s[at * 64 + 4 * n + (sub >> 2)] = (uint8_t)scale;
-      if (s_rows) s_rows[(size_t)b * 4 + (sub >> 2)] = (uint8_t)scale;
+      if (kRows && s_rows) s_rows[(size_t)b * 4 + (sub >> 2)] = (uint8_t)scale;
     }
   } else {
     if (sub == 0) {
       *reinterpret_cast<uint32_t*>(s + at * 64 + 4 * n) = scale;
-      if (s_rows) *reinterpret_cast<uint32_t*>(s_rows + (size_t)b * 4) = scale;
+      if (kRows && s_rows) *reinterpret_cast<uint32_t*>(s_rows + (size_t)b * 4) = scale;
     }
   }
-  if (q_rows) *reinterpret_cast<uint2*>(q_rows + (size_t)b * 128 + 8 * sub) = codes;
+  if (kRows && q_rows) *reinterpret_cast<uint2*>(q_rows + (size_t)b * 128 + 8 * sub) = codes;
 }
 
 struct Fp8Args {
@@ -321,9 +321,10 @@ __device__ __forceinline__ void row_mma(const RowChunk<TM, NT>& r, v4f (&acc)[NT
   }
 }
 
-// grid (ceil(tile sets / M), ceil(T / (16 NT)), K splits), 64 W threads. With more than one split a workgroup writes its
-// FP32 sums to a.partial (fp8_splitk_reduce_kernel adds them in split order).
-template <int kBlock, bool kFused, int W, int M, int TM, int NT, int P, bool kPair>
+// grid (ceil(tile sets / M), ceil(T / (16 NT)), kSplit: K splits), 64 W threads. kSplit: a workgroup writes its FP32 sums
+// to a.partial (fp8_splitk_reduce_kernel adds them in split order). A template argument: with the grid's size read in
+// every kernel the launches of a few us each took 0.2 us longer (shared expert of four layers 52.2 -> 53.7 us).
+template <int kBlock, bool kFused, int W, int M, int TM, int NT, int P, bool kPair, bool kSplit>
 __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
   static_assert(W % M == 0 && 4 * P * M <= kTileQRows && M * TM * NT <= W && (NT == 1 || !kFused) &&
                     (!kPair || (TM == 2 && NT == 1 && M == 1 && kBlock == 32)),
@@ -371,9 +372,10 @@ __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
   src.xs_chunk = a.ordered ? 64 : 4;
   // the workgroup's chunks: all of K, or its share of them (blockIdx.z of gridDim.z)
   int cb = 0, cw = C;
-  if (gridDim.z > 1) {
-    cb = (int)((int64_t)C * blockIdx.z / gridDim.z);
-    cw = (int)((int64_t)C * (blockIdx.z + 1) / gridDim.z) - cb;
+  if constexpr (kSplit) {
+    const int z = blockIdx.z, S = gridDim.z;   // at most 16: C z fits 32 bits
+    cb = C * z / S;
+    cw = C * (z + 1) / S - cb;
   }
   const int c0 = cb + (cw * kp) / KP, n = (cw * (kp + 1)) / KP - (cw * kp) / KP;
   // fused: K part kp's rows, block b = i ntok + token (chunk c0 + i), 128 codes + 16 bytes of padding each,
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(64 * W) void fp8_row_gemv_kernel(Fp8Args a) {
   const int local = 16 * (ft / TM) + nn;
   if (w >= M * TM * NT || local >= ntok || set_raw >= sets) return;
   const size_t o = (size_t)(tok0 + local) * a.N + 16 * (tile + ft % TM) + 4 * q;
-  if (gridDim.z > 1) {
+  if constexpr (kSplit) {
     *reinterpret_cast<float4*>(a.partial + (size_t)blockIdx.z * a.T * a.N + o) = o4;
     return;
   }
@@ -780,7 +782,7 @@ RowShape fp8_row_shape(int N, int K, int T) {
   const int tiles = N / 16, C = K / 128;
   if (C <= 4 && (tiles > 256 || T > kTok)) return {4, 4, 1};
   if (tiles <= 256) {
-    RowShape sh{fp8_fits(8, C, T) && (!fp8_fits(4, C, T) || (T <= 2 && C * T >= 48)) ? 8 : 4, 1, 1};
+    RowShape sh{fp8_fits(8, C, T) && (!fp8_fits(4, C, T) || (T <= 2 && C * T >= 56)) ? 8 : 4, 1, 1};
     // Where the tiles leave CUs idle and a part would run through more than 16 chunks, K is split over as many workgroups
     // as fill the 256 CUs, 32 chunks or more each, and a second launch adds the splits (about 2.5 us). Block 32, us without
     // / with, at 1 / 8 / 32 tokens: 512 x 12288 - / 10.8 -> 9.5 / 16.1 -> 11.9, 512 x 16384 - / 12.4 -> 9.7 / 19.0 -> 12.2,
@@ -822,7 +824,7 @@ int fp8_fused_passes(const RowShape& sh, int K, int T) {
 
 // fp8_row_gemv_kernel of shape (W, M, TM): P fused quantization passes, or P = 0 when x comes quantized. A combination
 // that fp8_row_shape does not make has no kernel and is an error, not a call that leaves y as it was.
-template <int kBlock, int W, int M, int TM, bool kPair = false>
+template <int kBlock, int W, int M, int TM, bool kPair = false, bool kSplit = false>
 int launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
   const int sets = kPair ? a.N / 16 : a.N / 16 / TM;
   auto go = [&](auto kernel, int tokens = kTok) {
@@ -836,23 +838,26 @@ int launch_row_gemv(const Fp8Args& a, int P, hipStream_t st, int S = 1) {
   // 11.1, 8 x 1024 12.8 and 14.7).
   if constexpr (W == 4 && M == 1)
     if (P == 0 && a.T > kTok && (a.ordered || a.N > 2048))
-      return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false>, 2 * kTok);
-  if (P == 0) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair>);
+      return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 2, 1, false, kSplit>, 2 * kTok);
+  if (P == 0) return go(fp8_row_gemv_kernel<kBlock, false, W, M, TM, 1, 1, kPair, kSplit>);
   if constexpr (W / M < 8 || kPair)   // 8 parts are only chosen for more blocks than one pass takes
-    if (P == 1) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair>);
+    if (P == 1) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 1, kPair, kSplit>);
   if constexpr (8 * M <= kTileQRows)
-    if (P == 2) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 2, kPair>);
+    if (P == 2) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 2, kPair, kSplit>);
   if constexpr (16 * M <= kTileQRows)
-    if (P == 4) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 4, kPair>);
+    if (P == 4) return go(fp8_row_gemv_kernel<kBlock, true, W, M, TM, 1, 4, kPair, kSplit>);
   return fail(MX_ERR_STATE, "FP8 GEMV: %d passes of the %d x %d x %d shape have no kernel", P, W, M, TM);
 }
 
 template <int kBlock>
 int launch_row_gemv(const RowShape& sh, const Fp8Args& a, int P, hipStream_t st) {
   const int shape = 100 * sh.W + 10 * sh.M + sh.TM;
-  if (sh.S > 1 && shape != 411) return fail(MX_ERR_STATE, "FP8 GEMV: shape %d does not split K", shape);
+  if (sh.S > 1) {
+    if (shape == 411) return launch_row_gemv<kBlock, 4, 1, 1, false, true>(a, P, st, sh.S);
+    return fail(MX_ERR_STATE, "FP8 GEMV: shape %d does not split K", shape);
+  }
   switch (shape) {
-    case 411: return launch_row_gemv<kBlock, 4, 1, 1>(a, P, st, sh.S);
+    case 411: return launch_row_gemv<kBlock, 4, 1, 1>(a, P, st);
     case 811: return launch_row_gemv<kBlock, 8, 1, 1>(a, P, st);
     case 412: return launch_row_gemv<kBlock, 4, 1, 2>(a, P, st);
     case 441: return launch_row_gemv<kBlock, 4, 4, 1>(a, P, st);
@@ -878,8 +883,10 @@ int launch_quant_ordered(int block, const uint16_t* x, uint8_t* q, void* s, int 
                          uint8_t* q_rows = nullptr, void* s_rows = nullptr) {
   const int C = K / 128;
   const dim3 grid((unsigned)(((int64_t)T * C + 15) / 16));
-  hipLaunchKernelGGL(block == 32 ? fp8_quant_ordered_kernel<32> : fp8_quant_ordered_kernel<128>, grid, dim3(256), 0, st, x,
-                     q, (uint8_t*)s, q_rows, (uint8_t*)s_rows, T, C);
+  const bool rows = q_rows || s_rows;
+  auto kernel = block == 32 ? (rows ? fp8_quant_ordered_kernel<32, true> : fp8_quant_ordered_kernel<32, false>)
+                            : (rows ? fp8_quant_ordered_kernel<128, true> : fp8_quant_ordered_kernel<128, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, x, q, (uint8_t*)s, q_rows, (uint8_t*)s_rows, T, C);
   MX_LAUNCH_CHECK("fp8_quant_ordered_kernel");
   return MX_OK;
 }
